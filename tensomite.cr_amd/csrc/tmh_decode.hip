@@ -356,7 +356,9 @@ __device__ __forceinline__ float fold_column(float acc, const float* pc, uint32_
 // (host.cr:408-440): q in l.q; keys and values of positions [0, n) in the
 // cache at kb/vb, but position `cur` (if ≥ 0) in l.kcur/l.vcur; positions
 // past `last` masked. Leaves the outputs in l.out. Every thread calls it.
-__device__ void attend(const AttLds& l, const float* __restrict__ kb, const float* __restrict__ vb, uint32_t width,
+// MAXM: the values a lane may hold for the total (ordered_sum_by_wave).
+template <int MAXM>
+__device__ __forceinline__ void attend(const AttLds& l, const float* __restrict__ kb, const float* __restrict__ vb, uint32_t width,
                        uint32_t n, int32_t last, int32_t cur, float scale) {
     __shared__ float tops[4];
     const uint32_t tid = threadIdx.x;
@@ -402,7 +404,7 @@ __device__ void attend(const AttLds& l, const float* __restrict__ kb, const floa
 
     for (uint32_t p = tid; p < n; p += 256u) l.sc[p] = maths_exp(l.sc[p] - top);
     __syncthreads();
-    const float total = shared_sum(l.sc, n);
+    const float total = shared_sum<MAXM>(l.sc, n);
     for (uint32_t p = tid; p < n; p += 256u) l.sc[p] = l.sc[p] / total;
     __syncthreads();
 
@@ -459,13 +461,11 @@ __device__ __forceinline__ void emit(const float* lout, float* out, uint32_t wid
     }
 }
 
-// One workgroup per (query token, head) of cached keys and values.
-__global__ __launch_bounds__(256) void k_attention(Attention a) {
-    extern __shared__ float4 lds4[];
-    const AttLds l = att_lds(reinterpret_cast<float*>(lds4), a.width, a.capacity);
+// The attention of token t, head h by the whole workgroup, from the
+// cached keys and values; an entry out of range gives zeros and a report.
+template <int MAXM>
+__device__ __forceinline__ void attend_one(const Attention& a, const AttLds& l, uint32_t t, uint32_t h) {
     const uint32_t tid = threadIdx.x;
-    const uint32_t t = blockIdx.x / a.heads;
-    const uint32_t h = blockIdx.x - t * a.heads;
     const int32_t row = a.table[3u * t], last = a.table[3u * t + 1u], length = a.table[3u * t + 2u];
     float* out = a.dst + (size_t)t * a.ld_dst + (size_t)h * a.width;
     if (row < 0 || row >= (int32_t)a.cache_rows || length <= 0 || length > (int32_t)a.capacity || last < 0 ||
@@ -479,14 +479,596 @@ __global__ __launch_bounds__(256) void k_attention(Attention a) {
     const float* qh = a.q + (size_t)t * a.ldq + (size_t)h * a.width;
     for (uint32_t c = tid; c < a.width; c += 256u) l.q[c] = qh[c];
     __syncthreads();
-    attend(l, a.keys + base, a.values + base, a.width, (uint32_t)length, last, -1, a.scale);
+    attend<MAXM>(l, a.keys + base, a.values + base, a.width, (uint32_t)length, last, -1, a.scale);
     emit(l.out, out, a.width, a.act, t, h, a.heads);
 }
 
-hipError_t launch_attention(const Attention& a, uint32_t tokens, hipStream_t stream) {
+// One workgroup per (query token, head).
+__global__ __launch_bounds__(256) void k_attention(Attention a) {
+    extern __shared__ float4 lds4[];
+    const uint32_t t = blockIdx.x / a.heads;
+    attend_one<128>(a, att_lds(reinterpret_cast<float*>(lds4), a.width, a.capacity), t, blockIdx.x - t * a.heads);
+}
+
+// The LDS float offset of key float f (position · width + column) of a chunk.
+__device__ __forceinline__ uint32_t att_key_at(uint32_t f) { return (f >> 8) * 260u + (f & 255u); }
+
+// Direct loads of the keys of positions [p0, p0 + cnt) into `to`, 1 KB a
+// load, 1040 bytes apart (att_key_at), loads wave, wave + WAVES, ...; returns
+// this wave's loads. Lanes past the chunk read its last piece again.
+template <uint32_t WAVES = 4>
+__device__ __forceinline__ uint32_t stage_keys(const float* kb, uint32_t width, uint32_t p0, uint32_t cnt,
+                                               uint32_t to, uint32_t wave) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uintptr_t base = (uintptr_t)(kb + (size_t)p0 * width);
+    const uintptr_t last = base + (uintptr_t)cnt * width * 4u - 16u;
+    const uint32_t loads = (cnt * width + 255u) >> 8;
+    uint32_t mine = 0;
+    for (uint32_t i = wave; i < loads; i += WAVES, ++mine) {
+        const uintptr_t a = base + (uintptr_t)i * 1024u + lane * 16u;
+        lds_load16((const void*)(a < last ? a : last), to + i * 1040u);
+    }
+    return mine;
+}
+
+// ------------------------------------------------------- prompt attention
+//
+// Tiles of up to 32 query rows of one head, for prompts: query rows of one
+// cache row that see different ends of the same positions. k_attention gives
+// each query row a workgroup that reads every key and value again and
+// computes masked positions too; here a key row is loaded once into the
+// registers of the lane that scores its position for all the tile's queries,
+// a value row once for all the queries of a wave, and masked positions are
+// left out. What bounds it is the arithmetic the host's rounding asks for: a
+// multiply and an add, separately rounded, per score column and per value
+// column (no fused or packed form has those bits). 512 tokens of 32 heads of
+// 64 take 65 us (469 with k_attention): 10 million wave multiplies and adds for
+// each of the two phases, 13 us at the rate DPP multiplies reach here (3.2
+// cycles an instruction with two waves a SIMD, 2.5 without DPP), ≈12 us of
+// exponentials and divisions, and the rest start, checks and barriers. With
+// scalar registers in DPP's place the scores waited for scalar loads; with a
+// key row loaded straight into each lane (64 rows a load) the loads took longer
+// than the arithmetic.
+//
+//   scores   keys stage through LDS 128 positions at a time (64 at width 128;
+//            direct loads, two buffers); a wave takes 64 positions for four queries, a lane a
+//            position with its key row in registers, a query's column
+//            reaching the lanes as the multiply's DPP operand (row_newbcast)
+//            from a register that holds 16 of them.
+//   softmax  each wave takes its own queries: top and Maths.exp across the
+//            lanes, then the totals as one chain of adds per query, a lane a
+//            query (all of a wave's totals for the price of one chain).
+//   values   a lane per column, the wave's queries' running sums in
+//            registers; 16 positions' weights of a query are one LDS read,
+//            multiplied by DPP likewise.
+//
+// Scores of a pass of `rows` queries lie in LDS; a tile whose positions leave
+// no room for all its queries runs in passes of fewer.
+//
+// Leaving a masked position out keeps the host's bits only where its score
+// is -inf (its exponential then +0, which leaves the total as it is) and its
+// value finite (its product then a zero, which leaves the sum as it is): each
+// tile checks the masked keys and values it would leave out (finite, and no
+// dot product able to overflow) and otherwise attends query by query as
+// k_attention does.
+
+// Query rows of a tile, at most; a workgroup's LDS at most (one workgroup of
+// eight waves a compute unit: two a SIMD, which the vector unit needs to issue
+// at its full rate).
+constexpr uint32_t TILE_ROWS = 32;
+constexpr uint32_t TILE_THREADS = 512, TILE_WAVES = TILE_THREADS / 64;
+constexpr size_t TILE_LDS = 156u * 1024u;
+
+// Positions staged at a time: two blocks of 64 where the keys' two buffers
+// leave room (head width 64), else one.
+__host__ __device__ constexpr uint32_t tile_blocks(uint32_t width) { return width == 64u ? 2u : 1u; }
+
+// Floats of a tile's LDS before its scores: two key buffers (att_key_at's
+// layout), then the queries.
+__host__ __device__ constexpr uint32_t tile_key_floats(uint32_t width) {
+    return tile_blocks(width) * (64u * width / 256u) * 260u;
+}
+__host__ __device__ constexpr uint32_t tile_fixed_floats(uint32_t width, uint32_t T) {
+    return 2u * tile_key_floats(width) + T * width;
+}
+
+// Lane i (0..15) of every 16-lane row's value, in all lanes of the row.
+template <int I>
+__device__ __forceinline__ float row_lane(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + I, 0xF, 0xF, true));
+}
+
+template <int Q, int C, int I = 0>
+__device__ __forceinline__ void add_positions(float (&acc)[Q][C], const float (&w)[Q], const float (&v)[16][C]) {
+    if constexpr (I < 16) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const float weight = row_lane<I>(w[q]);
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const float prod = weight * v[I][c];
+                acc[q][c] += prod;
+            }
+        }
+        add_positions<Q, C, I + 1>(acc, w, v);
+    }
+}
+
+// Wave-wide maximum of values that are no NaN, by DPP.
+__device__ __forceinline__ float wave_highest(float v) {
+#define TMH_STEP(ctrl, rows) \
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp((int)0xff800000, __float_as_int(v), ctrl, rows, 0xF, false)))
+    TMH_STEP(0x111, 0xF);
+    TMH_STEP(0x112, 0xF);
+    TMH_STEP(0x114, 0xF);
+    TMH_STEP(0x118, 0xF);
+    TMH_STEP(0x142, 0xA);
+    TMH_STEP(0x143, 0xC);
+#undef TMH_STEP
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
+// dot[i] += x[i] · k over W columns in order, N queries side by side (their
+// chains of adds overlap): lane c of every 16-lane row holds column 16·j + c of
+// query i in x[i][j], a lane's own k its position's columns.
+template <int W, int N, int I = 0>
+__device__ __forceinline__ void add_columns(float (&dot)[N], const float (&x)[N][W / 16], const float4 (&k)[W / 4]) {
+    if constexpr (I < W) {
+        const float4 k4 = k[I / 4];
+        const float kc = I % 4 == 0 ? k4.x : I % 4 == 1 ? k4.y : I % 4 == 2 ? k4.z : k4.w;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const float prod = row_lane<I % 16>(x[i][I / 16]) * kc;
+            dot[i] += prod;
+        }
+        add_columns<W, N, I + 1>(dot, x, k);
+    }
+}
+
+// A stage of a tile's scores: the keys of positions p0 ... in LDS, the pass's
+// queries, scores and the last position each query sees (lane l: query l).
+struct TileStage {
+    const float* keys;
+    const float* queries;
+    float* scores;
+    uint32_t S, p0;
+    int32_t seen;
+    uint32_t count;
+    float scale;
+};
+
+// The scores of a stage, dot products in column order, ·scale: a wave takes
+// units of a block of 64 positions (a lane a position, in an order whose
+// 16-byte reads of key rows fall on distinct banks: rows of a kilobyte
+// together, kilobytes 1040 bytes apart) and N queries side by side.
+template <int W, uint32_t N>
+__device__ __forceinline__ void tile_scores(const TileStage& s, uint32_t wave) {
+    constexpr uint32_t ROWS = 256u / W, STEP = 64u / ROWS, BLOCKS = tile_blocks(W);
+    const uint32_t lane = threadIdx.x & 63u, block = wave % BLOCKS;
+    const uint32_t pl = 64u * block + ROWS * (lane % STEP) + lane / STEP;
+    float4 k[W / 4];
+    bool loaded = false;
+    for (uint32_t q = N * (wave / BLOCKS); q < s.count; q += N * (TILE_WAVES / BLOCKS)) {
+        int32_t reach = -1;
+#pragma unroll
+        for (uint32_t i = 0; i < N; ++i) reach = max(reach, __builtin_amdgcn_readlane(s.seen, q + i));
+        if ((int32_t)(s.p0 + 64u * block) > reach) continue;
+        if (!loaded) {
+            const float4* k4 = reinterpret_cast<const float4*>(s.keys + att_key_at(pl * W));
+#pragma unroll
+            for (int c = 0; c < W / 4; ++c) k[c] = k4[c];
+            loaded = true;
+        }
+        constexpr uint32_t M = W == 64 ? N : 2u;  // what the registers hold beside a key row
+#pragma unroll
+        for (uint32_t i0 = 0; i0 < N; i0 += M) {
+            float x[M][W / 16], dot[M];
+#pragma unroll
+            for (uint32_t i = 0; i < M; ++i) {
+                dot[i] = 0.0f;
+#pragma unroll
+                for (int j = 0; j < W / 16; ++j) x[i][j] = s.queries[(q + i0 + i) * W + 16u * j + (lane & 15u)];
+            }
+            add_columns<W, M>(dot, x, k);
+            // (past a query's last position, and rows of no query: not read)
+#pragma unroll
+            for (uint32_t i = 0; i < M; ++i) s.scores[(q + i0 + i) * s.S + s.p0 + pl] = dot[i] * s.scale;
+        }
+    }
+}
+
+// Floats of a score row of n positions: whole stages, plus 4 (the totals'
+// 16-byte reads of up to 16 rows then fall on distinct banks).
+template <int W>
+__host__ __device__ constexpr uint32_t tile_row_floats(uint32_t n) {
+    constexpr uint32_t STAGE = 64u * tile_blocks(W);
+    return (n + STAGE - 1u) / STAGE * STAGE + 4u;
+}
+
+// What a tile's pass needs; S floats a score row.
+struct TilePass {
+    float* sc;
+    uint32_t S, t0, h;  // t0: the pass's first token
+};
+
+// The softmax and the values of the wave's Q queries (rows row0 ... of the
+// pass; `seen`: lane l holds the last position query row0 + l sees, -1 where
+// there is no such query).
+template <int W, int Q>
+__device__ __forceinline__ void tile_values(const Attention& a, const TilePass& s, uint32_t row0, int32_t seen, uint32_t tokens,
+                            const float* __restrict__ vb) {
+    constexpr int C = W / 64;
+    const uint32_t lane = threadIdx.x & 63u;
+    int32_t last = -1;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) last = max(last, __builtin_amdgcn_readlane(seen, q));
+    if (last < 0) return;
+    const uint32_t n = (uint32_t)last + 1u, n16 = (n + 15u) & ~15u;
+    float* rows = s.sc + row0 * s.S;
+    // 4 positions a lane, up to four queries' reads together
+    float4* rows4 = reinterpret_cast<float4*>(rows);
+    const uint32_t S4 = s.S >> 2;
+    constexpr int G = Q < 4 ? Q : 4;
+    for (int q0 = 0; q0 < Q; q0 += G) {
+        uint32_t mine[G];
+        float top[G];
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            mine[q] = (uint32_t)(__builtin_amdgcn_readlane(seen, q0 + q) + 1);
+            top[q] = -__builtin_inff();
+        }
+        for (uint32_t p = lane * 4u; p < n16; p += 256u) {
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+                const float4 x = rows4[(q0 + q) * S4 + (p >> 2)];
+                top[q] = p < mine[q] && x.x > top[q] ? x.x : top[q];
+                top[q] = p + 1u < mine[q] && x.y > top[q] ? x.y : top[q];
+                top[q] = p + 2u < mine[q] && x.z > top[q] ? x.z : top[q];
+                top[q] = p + 3u < mine[q] && x.w > top[q] ? x.w : top[q];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            top[q] = wave_highest(top[q]);
+            const float first = rows[(q0 + q) * s.S];
+            if (first != first) top[q] = first;  // the host's top is a NaN at position 0
+        }
+        for (uint32_t p = lane * 4u; p < n16; p += 256u) {
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+                float4 x = rows4[(q0 + q) * S4 + (p >> 2)];
+                x.x = p < mine[q] ? maths_exp(x.x - top[q]) : 0.0f;
+                x.y = p + 1u < mine[q] ? maths_exp(x.y - top[q]) : 0.0f;
+                x.z = p + 2u < mine[q] ? maths_exp(x.z - top[q]) : 0.0f;
+                x.w = p + 3u < mine[q] ? maths_exp(x.w - top[q]) : 0.0f;
+                rows4[(q0 + q) * S4 + (p >> 2)] = x;
+            }
+        }
+    }
+    asm volatile("" ::: "memory");  // (a wave's LDS operations take effect in order)
+    const float total = ordered_sum(rows + (lane % (uint32_t)Q) * s.S, n16);
+    for (int q0 = 0; q0 < Q; q0 += G) {
+        float t[G];
+#pragma unroll
+        for (int q = 0; q < G; ++q) t[q] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(total), q0 + q));
+        for (uint32_t p = lane * 4u; p < n16; p += 256u) {
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+                float4 x = rows4[(q0 + q) * S4 + (p >> 2)];
+                x.x = x.x / t[q];
+                x.y = x.y / t[q];
+                x.z = x.z / t[q];
+                x.w = x.w / t[q];
+                rows4[(q0 + q) * S4 + (p >> 2)] = x;
+            }
+        }
+    }
+    asm volatile("" ::: "memory");
+
+    float acc[Q][C];
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int c = 0; c < C; ++c) acc[q][c] = 0.0f;
+    const float* vl = vb + lane;
+    auto load = [&](float (&v)[16][C], uint32_t p0) {
+        if (p0 + 16u <= n) {
+            const float* vp = vl + (size_t)p0 * W;
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+#pragma unroll
+                for (int c = 0; c < C; ++c) v[i][c] = vp[i * W + 64 * c];
+        } else {
+            // rows past the last position: zeros, whose weights are zeros too
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+#pragma unroll
+                for (int c = 0; c < C; ++c) v[i][c] = p0 + i < n ? vl[(size_t)(p0 + i) * W + 64 * c] : 0.0f;
+        }
+    };
+    auto fold = [&](const float (&v)[16][C], uint32_t p0) {
+        float w[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) w[q] = rows[q * s.S + p0 + (lane & 15u)];
+        add_positions<Q, C>(acc, w, v);
+    };
+    float va[16][C], vc[16][C];
+    load(va, 0);
+    for (uint32_t p0 = 0; p0 < n16; p0 += 32u) {
+        const bool more = p0 + 16u < n16;
+        if (more) load(vc, p0 + 16u);
+        fold(va, p0);
+        if (more) {
+            if (p0 + 32u < n16) load(va, p0 + 32u);
+            fold(vc, p0 + 16u);
+        }
+    }
+
+    // the outputs, and their quantised blocks for the o product
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        float* out = a.dst + (size_t)(s.t0 + row0 + q) * a.ld_dst + (size_t)s.h * W;
+        if (__builtin_amdgcn_readlane(seen, q) >= 0) {
+#pragma unroll
+            for (int c = 0; c < C; ++c) out[lane + 64 * c] = acc[q][c];
+        }
+    }
+    if (!a.act.qs) return;
+    constexpr uint32_t BLOCKS = W / 32;
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int c = 0; c < C; ++c) rows[q * s.S + lane + 64 * c] = acc[q][c];
+    asm volatile("" ::: "memory");
+    const uint32_t k = a.heads * W, nb = k >> 5, sub = lane & 7u;
+    for (uint32_t g = lane >> 3; g < (uint32_t)Q * BLOCKS; g += 8u) {
+        const uint32_t q = g / BLOCKS, blk = g % BLOCKS;
+        const float4 v = *reinterpret_cast<const float4*>(rows + q * s.S + blk * 32u + sub * 4u);
+        const Q8Quad r = quantize_quad(v.x, v.y, v.z, v.w);
+        const size_t t = s.t0 + row0 + q;
+        if (t >= tokens) continue;
+        const uint32_t at = s.h * BLOCKS + blk;
+        *(uint32_t*)((int8_t*)a.act.qs + t * k + at * 32u + sub * 4u) = r.packed;
+        if (sub == 0) {
+            ((float*)a.act.scales)[t * nb + at] = r.scale;
+            ((float*)a.act.sums)[t * nb + at] = r.sum;
+            ((int32_t*)a.act.totals)[t * nb + at] = r.total;
+        }
+    }
+}
+
+// Whether token t's table entry names positions the cache holds, of the
+// cache row and the length that token `first`'s names.
+__device__ __forceinline__ bool entry_alike(const Attention& a, uint32_t t, uint32_t first) {
+    const int32_t row = a.table[3u * t], last = a.table[3u * t + 1u], length = a.table[3u * t + 2u];
+    return row == a.table[3u * first] && length == a.table[3u * first + 2u] && row >= 0 &&
+           row < (int32_t)a.cache_rows && length > 0 && length <= (int32_t)a.capacity && last >= 0 && last < length;
+}
+
+// The largest magnitudes' bits (a NaN's are above an infinity's) of `count`
+// floats at k and at v (a multiple of 4, 16-byte pieces), thread by thread.
+__device__ __forceinline__ void largest_bits(const float* __restrict__ k, const float* __restrict__ v, uint32_t count,
+                                             uint32_t& mk, uint32_t& mv) {
+    constexpr int U = 8;  // loads of each in flight
+    const uint4* k4 = reinterpret_cast<const uint4*>(k);
+    const uint4* v4 = reinterpret_cast<const uint4*>(v);
+    const uint32_t pieces = count >> 2;
+    mk = mv = 0;
+    for (uint32_t i0 = threadIdx.x; i0 < pieces; i0 += U * TILE_THREADS) {
+        uint4 x[U], y[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t i = min(i0 + TILE_THREADS * u, pieces - 1u);
+            x[u] = k4[i];
+            y[u] = v4[i];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            mk = max(mk, max(max(x[u].x & 0x7fffffffu, x[u].y & 0x7fffffffu), max(x[u].z & 0x7fffffffu, x[u].w & 0x7fffffffu)));
+            mv = max(mv, max(max(y[u].x & 0x7fffffffu, y[u].y & 0x7fffffffu), max(y[u].z & 0x7fffffffu, y[u].w & 0x7fffffffu)));
+        }
+    }
+}
+
+__device__ __forceinline__ uint32_t wave_max(uint32_t m) {
+#pragma unroll
+    for (int s = 32; s >= 1; s >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, s, 64));
+    return m;
+}
+
+// The attention of tokens [t0, t0 + count) (a tile of T), head h; false where a
+// masked key or value could reach the host's results, and nothing is written.
+// A tile whose tokens do not share a cache row and length (or hold an entry
+// out of range) is left alone. lds_floats: room for the scores.
+template <int W>
+__device__ __forceinline__ bool attend_tile(const Attention& a, float* lds, uint32_t lds_floats, uint32_t tokens,
+                                            uint32_t T, uint32_t t0, uint32_t count, uint32_t h) {
+    __shared__ uint32_t found[TILE_WAVES][3];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // lane l: the entry of the tile's token l
+    const uint32_t mine = t0 + min(lane, count - 1u);
+    const int32_t row = a.table[3u * mine], last = a.table[3u * mine + 1u], length = a.table[3u * mine + 2u];
+    const int32_t row0 = __builtin_amdgcn_readfirstlane(row), held = __builtin_amdgcn_readfirstlane(length);
+    if (__builtin_amdgcn_ballot_w64(!entry_alike(a, mine, t0)) != 0) return true;
+    const uint32_t kv = h / (a.heads / a.kv_heads);
+    const size_t base = ((size_t)row0 * a.kv_heads + kv) * a.capacity * W;
+    const float* kb = a.keys + base;
+    const float* vb = a.values + base;
+
+    // The masked positions: those some query does not see, up to the row's
+    // length.
+    int32_t least = last, most = last;
+#pragma unroll
+    for (int s = 32; s >= 1; s >>= 1) {
+        least = min(least, __shfl_xor(least, s, 64));
+        most = max(most, __shfl_xor(most, s, 64));
+    }
+    least = __builtin_amdgcn_readfirstlane(least);
+    most = __builtin_amdgcn_readfirstlane(most);
+    if (least + 1 < held) {
+        const uint32_t from = (uint32_t)(least + 1), masked = (uint32_t)held - from;
+        uint32_t mk, mv, mq = 0;
+        largest_bits(kb + (size_t)from * W, vb + (size_t)from * W, masked * W, mk, mv);
+        for (uint32_t i = tid; i < count * (uint32_t)W; i += TILE_THREADS)
+            mq = max(mq, __float_as_uint(a.q[(size_t)(t0 + i / W) * a.ldq + (size_t)h * W + i % W]) & 0x7fffffffu);
+        mk = wave_max(mk);
+        mv = wave_max(mv);
+        mq = wave_max(mq);
+        if (lane == 0) {
+            found[wave][0] = mk;
+            found[wave][1] = mv;
+            found[wave][2] = mq;
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t w = 0; w < TILE_WAVES; ++w) {
+            mk = max(mk, found[w][0]);
+            mv = max(mv, found[w][1]);
+            mq = max(mq, found[w][2]);
+        }
+        // no masked dot product, nor its product with the scale, can overflow
+        const float bound = __uint_as_float(mq) * __uint_as_float(mk) * (float)W;
+        const float scaled = bound * fabsf(a.scale);
+        if (!(mv < 0x7f800000u && bound < 1e38f && scaled < 1e38f)) return false;
+    }
+
+    const uint32_t S = tile_row_floats<W>((uint32_t)most + 1u);
+    uint32_t P = T;
+    while (P > 8u && P * S > lds_floats - tile_fixed_floats(W, T)) P >>= 1;
+    // the tile's queries (rows of none as the last)
+    for (uint32_t i = tid; i < T * (uint32_t)W; i += TILE_THREADS)
+        lds[2u * tile_key_floats(W) + i] = a.q[(size_t)(t0 + min(i / W, count - 1u)) * a.ldq + (size_t)h * W + i % W];
+    for (uint32_t q0 = 0; q0 < count; q0 += P) {
+        const uint32_t queries = min(P, count - q0);
+        // lane l: the last position query q0 + l sees
+        const int32_t seen_l = __shfl(last, (int)(q0 + lane < 64u ? q0 + lane : 63u), 64);
+        const int32_t seen = lane < queries ? seen_l : -1;
+        int32_t end = seen;
+#pragma unroll
+        for (int s = 32; s >= 1; s >>= 1) end = max(end, __shfl_xor(end, s, 64));
+        const uint32_t n = (uint32_t)__builtin_amdgcn_readfirstlane(end) + 1u;
+        float* scores = lds + tile_fixed_floats(W, T);
+        float* queries_lds = lds + 2u * tile_key_floats(W);
+        const TilePass pass{scores, S, t0 + q0, h};
+        constexpr uint32_t STAGE = 64u * tile_blocks(W);
+        lds_sync();  // the last pass's scores and keys (or the checks' loads) are done with
+        uint32_t ahead = stage_keys<TILE_WAVES>(kb, W, 0, min(STAGE, n), lds_address(lds), wave);
+        for (uint32_t p0 = 0, key = 0; p0 < n; p0 += STAGE, key ^= tile_key_floats(W)) {
+            // these positions' keys are in, the next ones' on their way
+            const uint32_t p1 = p0 + STAGE;
+            if (p1 < n) {
+                ahead = stage_keys<TILE_WAVES>(kb, W, p1, min(STAGE, n - p1),
+                                               lds_address(lds + (key ^ tile_key_floats(W))), wave);
+                wait_vm_lds_upto<8>(ahead);
+            } else {
+                wait_vm_lds<0>();
+            }
+            lds_sync();
+            const TileStage st{lds + key, queries_lds + q0 * W, scores, S, p0, seen, queries, a.scale};
+            if (P >= 16u)
+                tile_scores<W, 4>(st, wave);
+            else
+                tile_scores<W, 2>(st, wave);
+            lds_sync();  // the keys are read: their buffer may be filled again
+        }
+
+        // this wave's queries
+        const uint32_t per = P / TILE_WAVES, from = wave * per;
+        const int32_t seen_w = __shfl(seen, (int)min(from + lane, 63u), 64);
+        const int32_t own = lane < per ? seen_w : -1;
+        if (per == 4u)
+            tile_values<W, 4>(a, pass, from, own, tokens, vb);
+        else if (per == 2u)
+            tile_values<W, 2>(a, pass, from, own, tokens, vb);
+        else
+            tile_values<W, 1>(a, pass, from, own, tokens, vb);
+    }
+    return true;
+}
+
+// Workgroups [0, tiles · heads): a tile of T tokens (8, 16 or 32)
+// and a head; those after them attend the tokens of tiles that name more than
+// one cache row or length one by one.
+template <int W>
+__global__ __launch_bounds__(TILE_THREADS, 2) void k_attention_tile(Attention a, uint32_t tokens, uint32_t T, uint32_t tiles,
+                                                           uint32_t lds_floats) {
+    extern __shared__ float4 lds4[];
+    __shared__ uint32_t ragged;
+    float* lds = reinterpret_cast<float*>(lds4);
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, work = tiles * a.heads;
+    // query rows to attend one by one: every `step` from item to items (token
+    // item / heads, head item % heads)
+    uint32_t item, items, step;
+    const bool others = blockIdx.x >= work;
+    if (others) {
+        if (tid == 0) ragged = 0;
+        __syncthreads();
+        bool other = false;
+        for (uint32_t t = tid; t < tokens; t += TILE_THREADS) other = other || !entry_alike(a, t, t - t % T);
+        if (other) ragged = 1;
+        __syncthreads();
+        if (!ragged) return;
+        item = blockIdx.x - work;
+        items = tokens * a.heads;
+        step = gridDim.x - work;
+    } else {
+        const uint32_t h = blockIdx.x % a.heads, order = blockIdx.x / a.heads;
+        // a prompt's last tiles see most: they go first
+        const uint32_t t0 = (tiles - 1u - order) * T, count = min(T, tokens - t0);
+        if (attend_tile<W>(a, lds, lds_floats, tokens, T, t0, count, h)) return;
+        item = t0 * a.heads + h;
+        items = (t0 + count) * a.heads;
+        step = a.heads;
+    }
+    if (tid >= 256u) return;  // attend_one's threads
+    const AttLds l = att_lds(lds, W, a.capacity);
+    for (; item < items; item += step) {
+        const uint32_t t = item / a.heads, h = item - t * a.heads, first = t - t % T;
+        const uint32_t other = first + (lane < T ? lane : 0u);
+        // the workgroups after the tiles: tokens of whole tiles are not theirs
+        // (the same answer in every wave)
+        if (others && __builtin_amdgcn_ballot_w64(other < tokens && !entry_alike(a, other, first)) == 0) continue;
+        attend_one<32>(a, l, t, h);
+        __syncthreads();
+    }
+}
+
+// Fewest tokens the tiles take (a decode step's sequences are fewer, each with
+// a cache row of its own), and workgroups of k_attention a compute unit holds
+// at a time: up to one such round the tiles gain little and their longer
+// start costs (9 heads of 64, no past: 64 tokens 8.6 us against 9.2 in tiles,
+// 100 tokens 15.8 against 10.0; 32 heads: 16 tokens 6.9 against 7.7, 32 tokens
+// 11.7 against 8.3, 128 tokens 49 against 20, 512 tokens 469 against 65).
+// The tiles' 16-byte loads need the caches 16-byte aligned.
+constexpr uint32_t TILE_MIN_TOKENS = 16, ROUND_WGS = 3;
+
+hipError_t launch_attention(const Attention& a, uint32_t tokens, bool prompt, int compute_units, hipStream_t stream) {
     if (tokens == 0 || a.heads == 0) return hipSuccess;
     const size_t lds = attention_lds(a.width, a.capacity);
-    TMH_LAUNCH(k_attention, dim3(tokens * a.heads), dim3(256), lds, stream, a);
+    if (tokens < TILE_MIN_TOKENS || (uint64_t)tokens * a.heads < ROUND_WGS * (uint64_t)compute_units ||
+        (a.width != 64u && a.width != 128u) || (((uintptr_t)a.keys | (uintptr_t)a.values) & 15u) != 0) {
+        TMH_LAUNCH(k_attention, dim3(tokens * a.heads), dim3(256), lds, stream, a);
+        return hipGetLastError();
+    }
+    // tiles small enough that two of them fall to each compute unit, where
+    // the tokens allow it
+    const uint32_t full = 2u * (uint32_t)compute_units;
+    uint32_t T = TILE_ROWS;
+    while (T > 8u && (uint64_t)((tokens + T - 1u) / T) * a.heads < full) T >>= 1;
+    const uint32_t tiles = (tokens + T - 1u) / T, work = tiles * a.heads;
+    const size_t row = a.width == 64u ? tile_row_floats<64>(a.capacity) : tile_row_floats<128>(a.capacity);
+    const size_t fixed = tile_fixed_floats(a.width, T);
+    const size_t tile_lds = std::max(lds, std::min(TILE_LDS, (fixed + T * row) * sizeof(float)));
+    if ((fixed + 8u * row) * sizeof(float) > tile_lds) {  // no room for eight queries' scores
+        TMH_LAUNCH(k_attention, dim3(tokens * a.heads), dim3(256), lds, stream, a);
+        return hipGetLastError();
+    }
+    const uint32_t others = prompt ? 0u : std::min(tokens * a.heads, full);
+    const uint32_t floats = (uint32_t)(tile_lds / sizeof(float));
+    if (a.width == 64u)
+        TMH_LAUNCH(k_attention_tile<64>, dim3(work + others), dim3(TILE_THREADS), tile_lds, stream, a, tokens, T, tiles, floats);
+    else
+        TMH_LAUNCH(k_attention_tile<128>, dim3(work + others), dim3(TILE_THREADS), tile_lds, stream, a, tokens, T, tiles, floats);
     return hipGetLastError();
 }
 
@@ -541,8 +1123,6 @@ __host__ __device__ inline uint32_t att_key_stride(uint32_t width) { return widt
 __host__ __device__ inline uint32_t att_kt_floats(uint32_t width, uint32_t cp) {
     return ((cp * width + 255u) >> 8) * 260u;
 }
-// The LDS float offset of key float f (position · width + column) of a chunk.
-__device__ __forceinline__ uint32_t att_key_at(uint32_t f) { return (f >> 8) * 260u + (f & 255u); }
 __host__ __device__ inline uint32_t att_v_floats(uint32_t width, uint32_t cp) { return (cp * width + 255u) & ~255u; }
 
 __device__ __forceinline__ AttDecodeLds att_decode_lds(float* base, uint32_t width, uint32_t capacity) {
@@ -574,23 +1154,6 @@ __device__ __forceinline__ uint32_t stage_row(const float* src, uint32_t width, 
     for (uint32_t c0 = 0; c0 < width; c0 += 64u, ++loads)
         lds_load4(src + min(c0 + lane, width - 1u), to + c0 * 4u);
     return loads;
-}
-
-// Direct loads of the keys of positions [p0, p0 + cnt) into `to`, 1 KB a
-// load, 1040 bytes apart (att_key_at), loads wave, wave + 4, ...; returns
-// this wave's loads. Lanes past the chunk read its last piece again.
-__device__ __forceinline__ uint32_t stage_keys(const float* kb, uint32_t width, uint32_t p0, uint32_t cnt,
-                                               uint32_t to, uint32_t wave) {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uintptr_t base = (uintptr_t)(kb + (size_t)p0 * width);
-    const uintptr_t last = base + (uintptr_t)cnt * width * 4u - 16u;
-    const uint32_t loads = (cnt * width + 255u) >> 8;
-    uint32_t mine = 0;
-    for (uint32_t i = wave; i < loads; i += 4u, ++mine) {
-        const uintptr_t a = base + (uintptr_t)i * 1024u + lane * 16u;
-        lds_load16((const void*)(a < last ? a : last), to + i * 1040u);
-    }
-    return mine;
 }
 
 // Direct loads of the value rows of positions [p0, p0 + cnt) into `to` (as

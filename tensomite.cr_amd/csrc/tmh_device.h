@@ -334,11 +334,12 @@ __device__ __forceinline__ float ordered_sum_by_wave(const float* v, uint32_t n)
 }
 
 // The ordered sum of v[0..n) by wave 0 (ordered_sum_by_wave; beyond its
-// limit, ordered_sum), shared through LDS. Every thread calls it.
+// limit, ordered_sum), shared through LDS. Every thread calls it. MAXM as there.
+template <int MAXM = 128>
 __device__ __forceinline__ float shared_sum(const float* v, uint32_t n) {
     __shared__ float result;
     if (threadIdx.x < 64u) {
-        const float sum = n <= WAVE_SUM_MAX ? ordered_sum_by_wave(v, n) : ordered_sum(v, n);
+        const float sum = n <= 64u * MAXM ? ordered_sum_by_wave<false, MAXM>(v, n) : ordered_sum(v, n);
         if (threadIdx.x == 0) result = sum;
     }
     __syncthreads();

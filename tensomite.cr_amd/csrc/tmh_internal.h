@@ -289,7 +289,8 @@ struct Attention {
 };
 size_t attention_lds(uint32_t width, uint32_t capacity);
 size_t attention_decode_lds(uint32_t width, uint32_t capacity);  // of launch_attention_decode
-hipError_t launch_attention(const Attention& a, uint32_t tokens, hipStream_t stream);
+// `prompt`: every token is known to name the same cache row and length, in range.
+hipError_t launch_attention(const Attention& a, uint32_t tokens, bool prompt, int compute_units, hipStream_t stream);
 // A decode step's attention with the RoPE and cache write of `r` fused: each
 // token is its cache row's one new position.
 hipError_t launch_attention_decode(const Attention& a, const RopeWrite& r, uint32_t tokens, hipStream_t stream);

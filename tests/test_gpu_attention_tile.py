@@ -1,0 +1,112 @@
+"""Attention over many tokens (the prompt tiles) against the oracle, bit for
+bit: tile sizes 8, 16 and 32, partial tiles, a past, passes of fewer queries
+than a tile, head widths 64 and 128, tiles of several cache rows, and masked
+keys and values that reach the host's results."""
+import sys
+
+import numpy as np
+import pytest
+
+from oracle import oracle
+import tensomite_hip as th
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    return th.HIPDevice(0)
+
+
+def attend(dev, q, k, v, table):
+    tokens, heads, width = q.shape
+    rows, kv_heads, capacity, _ = k.shape
+    scale = float(np.float32(1.0 / np.sqrt(width)))
+    out = dev.attention(dev.from_array(q), tokens, heads, dev.from_array(k), dev.from_array(v), rows, kv_heads,
+                        capacity, width, dev.from_array(np.array(table, np.int32)), scale)
+    return dev.to_array(out, np.float32, q.size).reshape(q.shape), scale
+
+
+def same(got, want):
+    nan = np.isnan(want)
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(got.view(np.uint32)[~nan], want.view(np.uint32)[~nan])
+
+
+def inputs(seed, tokens, heads, kv_heads, width, capacity, rows=1):
+    rng = np.random.default_rng(seed)
+    cache = (rows, kv_heads, capacity, width)
+    q, k, v = (rng.normal(0, 1, s).astype(np.float32) for s in ((tokens, heads, width), cache, cache))
+    q[tokens // 2] *= 40.0  # sharp softmax: many exponentials underflow to 0
+    return q, k, v
+
+
+# tokens · heads from one round of workgroups up; tiles of 8, 16 and 32 tokens
+# (their count times heads against two a compute unit), whole and partial; the
+# last two: score rows too long for all a tile's queries, and one position
+@pytest.mark.parametrize("tokens,heads,kv_heads,width,past,capacity", [
+    (24, 32, 32, 64, 0, 24), (97, 9, 3, 64, 0, 512), (130, 8, 2, 64, 3, 140), (257, 32, 4, 64, 1, 300),
+    (512, 32, 32, 64, 0, 512), (100, 12, 4, 128, 30, 131), (330, 32, 2, 128, 0, 400), (160, 52, 4, 64, 1240, 1400),
+    (16, 48, 48, 64, 0, 2048)])
+def test_prompt_tiles(dev, tokens, heads, kv_heads, width, past, capacity):
+    print("prompt tiles", tokens, heads, kv_heads, width, past, capacity, flush=True)
+    q, k, v = inputs(tokens + past, tokens, heads, kv_heads, width, capacity)
+    table = [(0, past + t, past + tokens) for t in range(tokens)]
+    got, scale = attend(dev, q, k, v, table)
+    dev.sync()
+    same(got, oracle.attention(q, k, v, table, scale))
+
+
+def test_tiles_of_several_rows(dev):
+    # tokens 0-15 a whole tile, 16-39 each its own row and length, the rest
+    # of the second row; one row's ends in no order
+    tokens, heads, capacity = 72, 16, 90
+    q, k, v = inputs(5, tokens, heads, 4, 64, capacity, rows=3)
+    rng = np.random.default_rng(6)
+    table = [(0, int(rng.integers(0, 60)), 60) for _ in range(16)]
+    for t in range(16, 40):
+        length = int(rng.integers(1, capacity + 1))
+        table.append((t % 3, int(rng.integers(0, length)), length))
+    table += [(1, t, 80) for t in range(tokens - 40)]
+    got, scale = attend(dev, q, k, v, table)
+    dev.sync()
+    same(got, oracle.attention(q, k, v, table, scale))
+
+
+def test_tile_entry_out_of_range(dev):
+    # the entry's token gets zeros and a report, the others their attention
+    tokens, heads, capacity = 64, 16, 64
+    q, k, v = inputs(8, tokens, heads, 16, 64, capacity)
+    table = [(0, t, tokens) for t in range(tokens)]
+    good = oracle.attention(q, k, v, table, float(np.float32(0.125)))
+    table[37] = (0, 3, capacity + 1)
+    got, _ = attend(dev, q, k, v, table)
+    with pytest.raises(th.ExecutionError):
+        dev.sync()
+    assert np.all(got[37] == 0)
+    keep = np.arange(tokens) != 37
+    same(got[keep], good[keep])
+
+
+@pytest.mark.parametrize("poison", ["value nan", "value inf", "key nan", "key inf", "key huge", "seen nan", "query huge"])
+def test_masked_keys_and_values(dev, poison):
+    # the host's masked positions take part: a masked value that is not
+    # finite times a zero weight, a masked score that is NaN or +inf - inf
+    print("masked", poison, flush=True)
+    tokens, heads, capacity, past = 96, 16, 160, 40
+    q, k, v = inputs(11, tokens, heads, 8, 64, capacity)
+    at = past + 70  # masked for the first 70 tokens
+    if poison.startswith("value"):
+        v[0, 3, at, 5] = np.nan if poison.endswith("nan") else -np.inf
+    elif poison.startswith("key"):
+        k[0, 3, at, 5] = {"nan": np.nan, "inf": np.inf, "huge": 3e38}[poison.split()[1]]
+    elif poison == "seen nan":
+        k[0, 2, 0, 9] = np.nan
+        v[0, 5, 7, 1] = np.inf
+    else:
+        q[20, 4] *= np.float32(1e37)
+    table = [(0, past + t, past + tokens) for t in range(tokens)]
+    with np.errstate(all="ignore"):
+        got, scale = attend(dev, q, k, v, table)
+        dev.sync()
+        same(got, oracle.attention(q, k, v, table, scale))
