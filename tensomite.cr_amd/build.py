@@ -28,7 +28,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 LIB = os.path.join(HERE, "libtensomite_hip.so")
-SOURCES = [os.path.join(HERE, "csrc", name) for name in ("tmh_runtime.hip", "tmh_kernels.hip", "tmh_decode.hip", "tmh_llama.hip", "tmh_gguf.hip", "tmh_quant_host.hip")]
+SOURCES = [os.path.join(HERE, "csrc", name) for name in ("tmh_runtime.hip", "tmh_kernels.hip", "tmh_mx.hip", "tmh_decode.hip", "tmh_llama.hip", "tmh_gguf.hip", "tmh_quant_host.hip")]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 FLAGS = [

@@ -442,6 +442,15 @@ __device__ __forceinline__ void lds_load16(const void* from, uint32_t lds) {
     asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "{m0}"(lds) : "memory");
 }
 
+// lds_load16 of base + off, the base uniform. The compiler does not see that the
+// instruction reads the base's scalar registers as an address, so the waits it
+// would put after a vector instruction that wrote them (v_readlane, where a
+// spilled base comes back; five wait states before a memory instruction
+// reads them) stand here.
+__device__ __forceinline__ void lds_load16_at(const void* base, uint32_t off, uint32_t lds) {
+    asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(lds) : "memory");
+}
+
 // lds_load16 marked non-temporal: weights stream through the caches once,
 // so they should not displace what is read again (activations, tables).
 __device__ __forceinline__ void lds_load16_nt(const void* from, uint32_t lds) {

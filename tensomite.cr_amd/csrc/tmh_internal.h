@@ -53,6 +53,14 @@ struct Activations {
 hipError_t launch_quantize(const float* x, uint32_t ldx, uint32_t rows, uint32_t k, float* scales, float* sums,
                            int32_t* totals, int8_t* qs, hipStream_t stream);
 
+// The matrix-core kernels' workgroup tiles (rows x outputs) and which of them a
+// product takes; MX_64X64 is k_matmul_mx, the others launch_matmul_tiles
+// (k a multiple of 256, 16-byte aligned weights and activation parts).
+enum MxTile { MX_32X32, MX_64X64, MX_64X128, MX_128X128 };
+MxTile mx_tile(uint32_t rows, uint32_t n, int compute_units);
+hipError_t launch_matmul_tiles(uint32_t kind, MxTile tile, const uint8_t* w, Activations act, float* dst,
+                               const float* bias, uint32_t rows, uint32_t n, uint32_t k, hipStream_t stream);
+
 // Launches dst[rows, n] = x · wᵀ (+ bias) over quantised activations, in the
 // kernel `mode` asks for (TMH_MODE_*). `w` points at the first weight row.
 hipError_t launch_block_matmul(uint32_t kind, uint32_t mode, const uint8_t* w, Activations act, float* dst,

@@ -2084,7 +2084,8 @@ __global__ __launch_bounds__(MX_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
 
     if (producer) return;
     const uint32_t col = n0 + nw + l32;
-    const float b = (bias && col < n) ? bias[col] : 0.0f;
+    float b = (bias && col < n) ? bias[col] : 0.0f;
+    asm volatile("" : "+v"(b));  // waited for here, once: not before every store, with the stores before it
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         const uint32_t row = m0 + mw + 8u * (i / 4) + 4u * half + (i % 4);
@@ -3647,6 +3648,8 @@ hipError_t launch_block_matmul(uint32_t kind, uint32_t mode, const uint8_t* w, A
     // own order (tree_fold, set by the entry point)
     const bool autoish = mode == 0u /* AUTO */ || mode == 3u /* UNORDERED */;
     if ((matrix || fused) && mx_fits(w, act, kind, k)) {
+        const MxTile tile = fused ? MX_64X64 : mx_tile(rows, n, compute_units);
+        if (tile != MX_64X64) return launch_matmul_tiles(kind, tile, w, act, dst, bias, rows, n, k, stream);
         switch (kind) {
         case 0: return launch_mx<0>(fused, w, act, dst, bias, rows, n, k, stream);
         case 1: return launch_mx<1>(fused, w, act, dst, bias, rows, n, k, stream);
