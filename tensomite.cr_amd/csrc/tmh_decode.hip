@@ -1033,6 +1033,318 @@ __global__ __launch_bounds__(TILE_THREADS, 2) void k_attention_tile(Attention a,
     }
 }
 
+// ------------------------------------------------------- few query rows
+//
+// One query row and head a workgroup of eight waves, for launches of at most
+// one workgroup a compute unit (a decode step's sequences): what a compute unit
+// can pull from HBM bounds it, so its loads stay in flight throughout.
+//
+//   scores   each wave takes blocks of 4096 / W positions (every `kwaves`-th),
+//            the keys by direct loads into LDS of its own, no barriers
+//   softmax  top, Maths.exp and the divisions across the workgroup, the total
+//            by wave 0 (ordered_sum_by_wave)
+//   values   rounds of 8 · 4096 / W positions, a block a wave, read into
+//            registers (lane: its columns) two rounds ahead, the first two before
+//            the softmax (EARLY: capacities up to 2048, whose totals leave the
+//            registers); the waves form their products together and then add
+//            them in turn to the running sums handed on through LDS
+//
+// Eight sequences of 500 to 2001 positions, 32 heads of 64: 80.2 -> 49 us a launch (176
+// MB of keys and values: 3.6 TB/s); one of 2001 positions 64.6 -> 31, one of 201 with
+// 9 heads 11.4 -> 8.0. k_attention read a chunk of 64 positions at a time, a
+// round trip each.
+constexpr uint32_t ROWS_THREADS = 512, ROWS_WAVES = ROWS_THREADS / 64;
+constexpr size_t ROWS_LDS = 159u * 1024u;
+constexpr uint32_t ROWS_KEY_FLOATS = 16u * 260u;  // a block's keys: 16 KB, 1040 bytes a kilobyte
+
+// Floats before the key buffers: q, the outputs, and the scores in whole rounds.
+__host__ __device__ inline uint32_t rows_fixed_floats(uint32_t width, uint32_t capacity) {
+    const uint32_t round = ROWS_WAVES * (4096u / width);
+    return 2u * width + (capacity + round - 1u) / round * round;
+}
+
+// dot over W columns in order of a key row and the query, whose column 16·j + c
+// lane c of every 16-lane row holds in x[j].
+template <int W, int C4 = 0>
+__device__ __forceinline__ void add_key_columns(float& dot, const float (&x)[W / 16], const float4 (&k)[W / 4]) {
+    if constexpr (C4 < W / 4) {
+        const float p0 = row_lane<C4 * 4 % 16>(x[C4 / 4]) * k[C4].x;
+        dot += p0;
+        const float p1 = row_lane<C4 * 4 % 16 + 1>(x[C4 / 4]) * k[C4].y;
+        dot += p1;
+        const float p2 = row_lane<C4 * 4 % 16 + 2>(x[C4 / 4]) * k[C4].z;
+        dot += p2;
+        const float p3 = row_lane<C4 * 4 % 16 + 3>(x[C4 / 4]) * k[C4].w;
+        dot += p3;
+        add_key_columns<W, C4 + 1>(dot, x, k);
+    }
+}
+
+// ROPE (a decode step): token t is its cache row's one new position (slot = row
+// · capacity + position, table (row, position, position + 1)); q and the new key
+// are rotated here from the qkv row, and the group's first head writes the new
+// key and value into the caches, which the others do not read there.
+template <int W, bool EARLY, bool ROPE>
+__global__ __launch_bounds__(ROWS_THREADS, 2) void k_attention_rows(Attention a, RopeWrite r, uint32_t kwaves) {
+    extern __shared__ float4 lds4[];
+    __shared__ float tops[ROWS_WAVES];
+    __shared__ float total_slot, first_slot;
+    constexpr uint32_t P = 4096u / W, C = W / 64;  // positions of a block; a lane's columns
+    float* lds = reinterpret_cast<float*>(lds4);
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t t = blockIdx.x / a.heads, h = blockIdx.x - t * a.heads;
+    const int32_t row = a.table[3u * t], last = a.table[3u * t + 1u], length = a.table[3u * t + 2u];
+    float* out = a.dst + (size_t)t * a.ld_dst + (size_t)h * W;
+    const int32_t slot = ROPE ? r.slots[t] : 0, cap = (int32_t)a.capacity;
+    const bool bad = ROPE ? slot < 0 || slot >= (int32_t)a.cache_rows * cap || row != slot / cap || last != slot % cap ||
+                                length != last + 1
+                          : row < 0 || row >= (int32_t)a.cache_rows || length <= 0 || length > cap || last < 0 ||
+                                last >= length;
+    if (bad) {
+        for (uint32_t c = tid; c < (uint32_t)W; c += ROWS_THREADS) out[c] = 0.0f;
+        if (tid == 0 && h == 0) {
+            if (ROPE) report(a.errors, slot, (int32_t)a.cache_rows * cap);
+            else report(a.errors, row < 0 || row >= (int32_t)a.cache_rows ? row : length, cap);
+        }
+        return;
+    }
+    const uint32_t n = (uint32_t)length, kv = h / (a.heads / a.kv_heads);
+    const size_t base = ((size_t)row * a.kv_heads + kv) * a.capacity * W;
+    const float* kb = a.keys + base;
+    const float* vb = a.values + base;
+    float* sums = lds;  // the running sums, then the outputs
+    float* sc = lds + 2u * W;
+    float* keys = lds + rows_fixed_floats(W, a.capacity) + wave * ROWS_KEY_FLOATS;
+
+    // ROPE: the new position's value row and rotated key (columns 64·c + lane)
+    const uint32_t held = ROPE ? n - 1u : n;  // positions the caches hold
+    float vnew[C], knew[C];
+    const float* qkv = ROPE ? r.x + (size_t)t * r.ldx : nullptr;
+    const float* cs = ROPE ? r.cos + (size_t)held * W : nullptr;
+    const float* sn = ROPE ? r.sin + (size_t)held * W : nullptr;
+    // What a column of q or of the new key is made of: its own and its partner's
+    // values and the tables', x·cos + (partner·-1 or partner)·sin (host.cr:448-466)
+    struct Column {
+        float own, partner, cos, sin;
+    };
+    auto column = [&](const float* head, uint32_t c) {
+        return Column{head[c], head[c < W / 2u ? c + W / 2u : c - W / 2u], cs[c], sn[c]};
+    };
+    auto rotated = [](const Column& v, uint32_t c) {
+        const float turned = c < W / 2u ? v.partner * -1.0f : v.partner;
+        const float left = v.own * v.cos, right = turned * v.sin;
+        return left + right;
+    };
+    // Everything the start reads goes out at once: the query's columns (and the
+    // new key's and value's), the wave's first keys, its first values.
+    float x[W / 16];
+    Column qc[W / 16], kc[C];
+#pragma unroll
+    for (int j = 0; j < W / 16; ++j) {
+        const uint32_t c = 16u * j + (lane & 15u);
+        if constexpr (ROPE) qc[j] = column(qkv + (size_t)h * W, c);
+        else x[j] = a.q[(size_t)t * a.ldq + (size_t)h * W + c];
+    }
+    if constexpr (ROPE) {
+#pragma unroll
+        for (uint32_t c = 0; c < C; ++c) {
+            vnew[c] = qkv[(size_t)(a.heads + a.kv_heads + kv) * W + 64u * c + lane];
+            kc[c] = column(qkv + (size_t)(a.heads + kv) * W, 64u * c + lane);
+        }
+    }
+    if (wave < kwaves && wave * P < n) stage_keys<1>(kb, W, wave * P, min(P, n - wave * P), lds_address(keys), 0);
+
+    // a block of values in registers: rows past those the cache holds zeros
+    auto load = [&](float (&v)[P][C], uint32_t p0) {
+        const float* vp = vb + (size_t)p0 * W + lane;
+#pragma unroll
+        for (uint32_t g = 0; g < P; g += 16u) {
+            if (p0 + g + 16u <= held) {
+#pragma unroll
+                for (uint32_t i = g; i < g + 16u; ++i)
+#pragma unroll
+                    for (uint32_t c = 0; c < C; ++c) v[i][c] = vp[(size_t)i * W + 64u * c];
+            } else if (p0 + g < held) {
+#pragma unroll
+                for (uint32_t i = g; i < g + 16u; ++i)
+#pragma unroll
+                    for (uint32_t c = 0; c < C; ++c) v[i][c] = p0 + i < held ? vp[(size_t)i * W + 64u * c] : 0.0f;
+            } else {
+#pragma unroll
+                for (uint32_t i = g; i < g + 16u; ++i)
+#pragma unroll
+                    for (uint32_t c = 0; c < C; ++c) v[i][c] = 0.0f;
+            }
+        }
+    };
+    constexpr uint32_t ROUND = ROWS_WAVES * P;
+    float va[P][C], vc[P][C];
+
+    constexpr bool FIRST = EARLY && W == 64;  // (a key row of 128 takes the registers)
+    if constexpr (FIRST) {
+        if (wave * P < held) load(va, wave * P);
+    }
+    if constexpr (ROPE) {
+#pragma unroll
+        for (int j = 0; j < W / 16; ++j) x[j] = rotated(qc[j], 16u * j + (lane & 15u));
+#pragma unroll
+        for (uint32_t c = 0; c < C; ++c) knew[c] = rotated(kc[c], 64u * c + lane);
+        if (h % (a.heads / a.kv_heads) == 0 && wave == ROWS_WAVES - 1u) {
+#pragma unroll
+            for (uint32_t c = 0; c < C; ++c) {
+                r.keys[base + (size_t)held * W + 64u * c + lane] = knew[c];
+                r.values[base + (size_t)held * W + 64u * c + lane] = vnew[c];
+            }
+        }
+    }
+
+    // scores
+    float top = -__builtin_inff();
+    if (wave < kwaves) {
+        // lane -> position of the block: 16-byte reads of key rows on distinct banks (tile_scores)
+        constexpr uint32_t ROWS = 256u / W, STEP = P / ROWS;
+        const uint32_t pl = lane < P ? ROWS * (lane % STEP) + lane / STEP : 0u;
+        for (uint32_t p0 = wave * P; p0 < n; p0 += kwaves * P) {
+            if (p0 != wave * P) stage_keys<1>(kb, W, p0, min(P, n - p0), lds_address(keys), 0);
+            // the first keys' loads stand before a whole block's value loads (64)
+            if (FIRST && p0 == wave * P && p0 + P <= held)
+                wait_vm_lds<63>();
+            else
+                wait_vm_lds<0>();
+            asm volatile("" ::: "memory");
+            if constexpr (ROPE) {
+                // the new position's key, not yet in what was staged (a wave's LDS operations take effect in order)
+                if (held - p0 < P) {
+#pragma unroll
+                    for (uint32_t c = 0; c < C; ++c) keys[att_key_at((held - p0) * W + 64u * c + lane)] = knew[c];
+                }
+                asm volatile("" ::: "memory");
+            }
+            const float4* k4 = reinterpret_cast<const float4*>(keys + att_key_at(pl * W));
+            float4 k[W / 4];
+#pragma unroll
+            for (int c = 0; c < W / 4; ++c) k[c] = k4[c];
+            float dot = 0.0f;
+            add_key_columns<W>(dot, x, k);
+            const uint32_t p = p0 + pl;
+            float s = dot * a.scale;
+            // The causal mask adds -inf past the last position seen; its 0
+            // elsewhere only turns a -0 score into +0, which changes no later bit.
+            if ((int32_t)p > last) s = s + -__builtin_inff();
+            if (lane < P && p < n) {
+                sc[p] = s;
+                top = s > top ? s : top;
+                if (p == 0) first_slot = s;
+            }
+            asm volatile("" ::: "memory");
+            wait_vm_lds<63>();  // the keys are read: the next ones may land
+        }
+    }
+    if constexpr (EARLY) {
+        if (!FIRST && wave * P < held) load(va, wave * P);
+        if (ROUND + wave * P < held) load(vc, ROUND + wave * P);
+    }
+    top = wave_highest(top);
+    if (lane == 0) tops[wave] = top;
+    lds_sync();
+    top = tops[0];
+#pragma unroll
+    for (uint32_t w = 1; w < ROWS_WAVES; ++w) top = tops[w] > top ? tops[w] : top;
+    if (first_slot != first_slot) top = first_slot;  // the host's top is a NaN at position 0
+    const uint32_t padded = (n + ROUND - 1u) / ROUND * ROUND;
+    for (uint32_t p = tid; p < padded; p += ROWS_THREADS) sc[p] = p < n ? maths_exp(sc[p] - top) : 0.0f;
+    lds_sync();
+    if (wave == 0) {
+        constexpr int MAXM = EARLY ? 32 : 128;
+        const float sum = n <= 64u * MAXM ? ordered_sum_by_wave<false, MAXM>(sc, n) : ordered_sum(sc, n);
+        if (lane == 0) total_slot = sum;
+    }
+    if constexpr (!EARLY) {
+        if (wave * P < held) load(va, wave * P);
+        if (ROUND + wave * P < held) load(vc, ROUND + wave * P);
+    }
+    lds_sync();
+    const float total = total_slot;
+    // each wave the weights of its own blocks
+    for (uint32_t p0 = wave * P; p0 < n; p0 += ROUND)
+        if (lane < P) sc[p0 + lane] = sc[p0 + lane] / total;
+    asm volatile("" ::: "memory");  // (a wave's LDS operations take effect in order)
+
+    // A round's products together, then wave after wave its chain of adds.
+    auto fold = [&](float (&v)[P][C], uint32_t r0) {
+        const uint32_t p0 = r0 + wave * P;
+        if (p0 < held) {
+#pragma unroll
+            for (uint32_t i = 0; i < P; i += 4u) {
+                const float4 w4 = *reinterpret_cast<const float4*>(sc + p0 + i);
+#pragma unroll
+                for (uint32_t c = 0; c < C; ++c) {
+                    v[i][c] = w4.x * v[i][c];
+                    v[i + 1u][c] = w4.y * v[i + 1u][c];
+                    v[i + 2u][c] = w4.z * v[i + 2u][c];
+                    v[i + 3u][c] = w4.w * v[i + 3u][c];
+                }
+            }
+        }
+        for (uint32_t w = 0; w < ROWS_WAVES && r0 + w * P < held; ++w) {
+            if (wave == w) {
+                float acc[C];
+#pragma unroll
+                for (uint32_t c = 0; c < C; ++c) acc[c] = p0 == 0 ? 0.0f : sums[lane + 64u * c];
+#pragma unroll
+                for (uint32_t i = 0; i < P; ++i)
+#pragma unroll
+                    for (uint32_t c = 0; c < C; ++c) acc[c] += v[i][c];
+#pragma unroll
+                for (uint32_t c = 0; c < C; ++c) sums[lane + 64u * c] = acc[c];
+                if (p0 + 2u * ROUND < held) load(v, p0 + 2u * ROUND);
+            }
+            lds_sync();
+        }
+    };
+    for (uint32_t r0 = 0; r0 < held; r0 += 2u * ROUND) {
+        fold(va, r0);
+        if (r0 + ROUND < held) fold(vc, r0 + ROUND);
+    }
+    if constexpr (ROPE) {
+        // the new position last
+        if (wave == 0) {
+#pragma unroll
+            for (uint32_t c = 0; c < C; ++c) {
+                const float prod = sc[held] * vnew[c];
+                sums[64u * c + lane] = (held ? sums[64u * c + lane] : 0.0f) + prod;
+            }
+        }
+        lds_sync();
+    }
+    emit(sums, out, W, a.act, t, h, a.heads);
+}
+
+// Head widths 64 and 128, at most a workgroup a compute unit (each takes its
+// LDS), and caches aligned for the keys' direct loads of 16 bytes.
+static bool rows_fits(const Attention& a, uint32_t tokens, int compute_units) {
+    return (((uintptr_t)a.keys | (uintptr_t)a.values) & 15u) == 0 && (a.width == 64u || a.width == 128u) &&
+           (uint64_t)tokens * a.heads <= (uint64_t)compute_units;
+}
+
+template <bool ROPE>
+static hipError_t launch_rows(const Attention& a, const RopeWrite& r, uint32_t tokens, hipStream_t stream) {
+    const size_t fixed = rows_fixed_floats(a.width, a.capacity) * sizeof(float), block = ROWS_KEY_FLOATS * sizeof(float);
+    const uint32_t kwaves = (uint32_t)std::min<size_t>(ROWS_WAVES, (ROWS_LDS - fixed) / block);
+    const size_t lds = fixed + kwaves * block;
+    const dim3 grid(tokens * a.heads), threads(ROWS_THREADS);
+    const bool early = a.capacity <= 2048u;
+    if (a.width == 64u && early)
+        TMH_LAUNCH((k_attention_rows<64, true, ROPE>), grid, threads, lds, stream, a, r, kwaves);
+    else if (a.width == 64u)
+        TMH_LAUNCH((k_attention_rows<64, false, ROPE>), grid, threads, lds, stream, a, r, kwaves);
+    else if (early)
+        TMH_LAUNCH((k_attention_rows<128, true, ROPE>), grid, threads, lds, stream, a, r, kwaves);
+    else
+        TMH_LAUNCH((k_attention_rows<128, false, ROPE>), grid, threads, lds, stream, a, r, kwaves);
+    return hipGetLastError();
+}
+
 // Fewest tokens the tiles take (a decode step's sequences are fewer, each with
 // a cache row of its own), and workgroups of k_attention a compute unit holds
 // at a time: up to one such round the tiles gain little and their longer
@@ -1045,8 +1357,10 @@ constexpr uint32_t TILE_MIN_TOKENS = 16, ROUND_WGS = 3;
 hipError_t launch_attention(const Attention& a, uint32_t tokens, bool prompt, int compute_units, hipStream_t stream) {
     if (tokens == 0 || a.heads == 0) return hipSuccess;
     const size_t lds = attention_lds(a.width, a.capacity);
+    const bool aligned = (((uintptr_t)a.keys | (uintptr_t)a.values) & 15u) == 0;
+    if (rows_fits(a, tokens, compute_units)) return launch_rows<false>(a, RopeWrite{}, tokens, stream);
     if (tokens < TILE_MIN_TOKENS || (uint64_t)tokens * a.heads < ROUND_WGS * (uint64_t)compute_units ||
-        (a.width != 64u && a.width != 128u) || (((uintptr_t)a.keys | (uintptr_t)a.values) & 15u) != 0) {
+        (a.width != 64u && a.width != 128u) || !aligned) {
         TMH_LAUNCH(k_attention, dim3(tokens * a.heads), dim3(256), lds, stream, a);
         return hipGetLastError();
     }
@@ -1491,8 +1805,10 @@ __global__ __launch_bounds__(256) void k_attention_decode(Attention a, RopeWrite
     emit(l.out, out, width, a.act, t, h, a.heads);
 }
 
-hipError_t launch_attention_decode(const Attention& a, const RopeWrite& r, uint32_t tokens, hipStream_t stream) {
+hipError_t launch_attention_decode(const Attention& a, const RopeWrite& r, uint32_t tokens, int compute_units,
+                                   hipStream_t stream) {
     if (tokens == 0 || a.heads == 0) return hipSuccess;
+    if (rows_fits(a, tokens, compute_units)) return launch_rows<true>(a, r, tokens, stream);
     const size_t lds = attention_decode_lds(a.width, a.capacity);
     TMH_LAUNCH(k_attention_decode, dim3(tokens * a.heads), dim3(256), lds, stream, a, r);
     return hipGetLastError();

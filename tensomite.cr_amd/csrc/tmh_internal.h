@@ -301,7 +301,8 @@ size_t attention_decode_lds(uint32_t width, uint32_t capacity);  // of launch_at
 hipError_t launch_attention(const Attention& a, uint32_t tokens, bool prompt, int compute_units, hipStream_t stream);
 // A decode step's attention with the RoPE and cache write of `r` fused: each
 // token is its cache row's one new position.
-hipError_t launch_attention_decode(const Attention& a, const RopeWrite& r, uint32_t tokens, hipStream_t stream);
+hipError_t launch_attention_decode(const Attention& a, const RopeWrite& r, uint32_t tokens, int compute_units,
+                                   hipStream_t stream);
 
 // RMSNorm then quantisation into `act`, one launch; for n a multiple of 32
 // up to the LDS limit.

@@ -173,8 +173,9 @@ hipError_t residual(const Llama& m, const DeviceContext& ctx, const uint8_t* w, 
 // The forward of `tokens` ids already on the device (m.ids), whose slots
 // and attention entries are on the device too; then the final norm and the
 // head over `final_rows` rows from row `final_from`, into logits rows from
-// `logits_row`. With `decode`, token t is cache row t's one new position, and
-// its RoPE and cache write run inside the attention launch.
+// `logits_row`. With `decode`, every token is its cache row's one new position
+// (a decode step, or a forward of one id), and its RoPE and cache write run
+// inside the attention launch.
 hipError_t forward_tokens(const Llama& m, const DeviceContext& ctx, uint32_t tokens, uint32_t final_from,
                           uint32_t final_rows, uint32_t logits_row, bool decode) {
     const tmh::TreeFold order(m.mode == TMH_MODE_UNORDERED);
@@ -215,7 +216,7 @@ hipError_t forward_tokens(const Llama& m, const DeviceContext& ctx, uint32_t tok
                          quant_att ? a_att : tmh::Activations{}};
         if (e == hipSuccess) {
             if (decode) {
-                e = tmh::launch_attention_decode(a, r, tokens, ctx.stream);
+                e = tmh::launch_attention_decode(a, r, tokens, ctx.compute_units, ctx.stream);
             } else {
                 e = tmh::launch_rope_write(r, tokens, ctx.stream);
                 if (e == hipSuccess) e = tmh::launch_attention(a, tokens, true, ctx.compute_units, ctx.stream);
@@ -607,7 +608,7 @@ int tmh_llama_forward(uint64_t model, uint32_t row, const int32_t* ids, uint32_t
     // generation starts from.
     const uint32_t logits_row = last_only ? row : 0u;
     if (e == hipSuccess)
-        e = forward_tokens(*m, ctx, count, last_only ? count - 1u : 0u, final_rows, logits_row, false);
+        e = forward_tokens(*m, ctx, count, last_only ? count - 1u : 0u, final_rows, logits_row, count == 1u);
     if (e != hipSuccess) return code(e);
     tmh::note_launch(ctx.index, 0, true);
     m->length[row] = past + (int32_t)count;

@@ -110,3 +110,50 @@ def test_masked_keys_and_values(dev, poison):
         got, scale = attend(dev, q, k, v, table)
         dev.sync()
         same(got, oracle.attention(q, k, v, table, scale))
+
+
+# One workgroup a query row and head: positions of one, two and more rounds of
+# value blocks, whole and partial blocks, capacities on both sides of 2048, few
+# and many heads; the last past the causal end (masked positions).
+@pytest.mark.parametrize("width", [64, 128])
+@pytest.mark.parametrize("capacity,lengths", [
+    (70, [1, 63, 64, 65, 70]), (600, [128, 129, 511, 512, 513, 600]), (1100, [1024, 1025, 1040, 1100]),
+    (2048, [2048, 1537, 16]), (3000, [3000, 2049, 17]), (5200, [5200])])
+def test_few_query_rows(dev, width, capacity, lengths):
+    print("few rows", width, capacity, lengths, flush=True)
+    heads, kv_heads = 4, 2
+    q, k, v = inputs(capacity + width, len(lengths), heads, kv_heads, width, capacity, rows=len(lengths))
+    for seen in (1.0, 0.6):
+        table = [(i, max(0, int(n * seen) - 1), n) for i, n in enumerate(lengths)]
+        got, scale = attend(dev, q, k, v, table)
+        dev.sync()
+        same(got, oracle.attention(q, k, v, table, scale))
+    k[0, 0, 0, 3] = np.nan  # a NaN at position 0 reaches every weight of its head
+    v[-1, 1, lengths[-1] - 1, 2] = np.inf
+    table = [(i, n - 1, n) for i, n in enumerate(lengths)]
+    with np.errstate(all="ignore"):
+        got, scale = attend(dev, q, k, v, table)
+        dev.sync()
+        same(got, oracle.attention(q, k, v, table, scale))
+
+
+@pytest.mark.parametrize("head_width,capacity", [(64, 1200), (128, 700), (64, 2600)])
+def test_decode_past_several_rounds(dev, head_width, capacity):
+    # the decode step's form (RoPE, the cache write and the new position
+    # inside): one-id forwards after a long prompt against one forward
+    from llama_fixtures import random_llama
+    config = dict(layers=1, width=128, heads=4, kv_heads=2, head_width=head_width, hidden=64, vocab=64,
+                  context=capacity, eps=1e-5, theta=10000.0, kind="Q8_0")
+    weights = random_llama(config, seed=capacity, std=0.2)
+    ids = np.random.default_rng(3).integers(0, 64, capacity).astype(np.int32)
+    want = oracle.Llama(config, weights).forward([int(i) for i in ids])
+    model = th.HIPLlama(dev, config, weights, max_tokens=512)
+    at = 0
+    for upto in [u for u in (0, 60, 63, 127, 511, 513, 1023, 1025) if u < capacity - 3] + [capacity - 2]:
+        if upto > at:
+            model.forward(ids[at:upto], last_only=True)
+            at = upto
+        for _ in range(2):
+            got = model.forward(ids[at:at + 1])
+            assert np.array_equal(got.view(np.uint32)[0], want.view(np.uint32)[at]), at
+            at += 1
