@@ -356,8 +356,6 @@ __device__ __forceinline__ float fold_column(float acc, const float* pc, uint32_
 // (host.cr:408-440): q in l.q; keys and values of positions [0, n) in the
 // cache at kb/vb, but position `cur` (if ≥ 0) in l.kcur/l.vcur; positions
 // past `last` masked. Leaves the outputs in l.out. Every thread calls it.
-// MAXM: the values a lane may hold for the total (ordered_sum_by_wave).
-template <int MAXM>
 __device__ __forceinline__ void attend(const AttLds& l, const float* __restrict__ kb, const float* __restrict__ vb, uint32_t width,
                        uint32_t n, int32_t last, int32_t cur, float scale) {
     __shared__ float tops[4];
@@ -404,7 +402,7 @@ __device__ __forceinline__ void attend(const AttLds& l, const float* __restrict_
 
     for (uint32_t p = tid; p < n; p += 256u) l.sc[p] = maths_exp(l.sc[p] - top);
     __syncthreads();
-    const float total = shared_sum<MAXM>(l.sc, n);
+    const float total = shared_sum(l.sc, n);
     for (uint32_t p = tid; p < n; p += 256u) l.sc[p] = l.sc[p] / total;
     __syncthreads();
 
@@ -463,7 +461,6 @@ __device__ __forceinline__ void emit(const float* lout, float* out, uint32_t wid
 
 // The attention of token t, head h by the whole workgroup, from the
 // cached keys and values; an entry out of range gives zeros and a report.
-template <int MAXM>
 __device__ __forceinline__ void attend_one(const Attention& a, const AttLds& l, uint32_t t, uint32_t h) {
     const uint32_t tid = threadIdx.x;
     const int32_t row = a.table[3u * t], last = a.table[3u * t + 1u], length = a.table[3u * t + 2u];
@@ -479,7 +476,7 @@ __device__ __forceinline__ void attend_one(const Attention& a, const AttLds& l, 
     const float* qh = a.q + (size_t)t * a.ldq + (size_t)h * a.width;
     for (uint32_t c = tid; c < a.width; c += 256u) l.q[c] = qh[c];
     __syncthreads();
-    attend<MAXM>(l, a.keys + base, a.values + base, a.width, (uint32_t)length, last, -1, a.scale);
+    attend(l, a.keys + base, a.values + base, a.width, (uint32_t)length, last, -1, a.scale);
     emit(l.out, out, a.width, a.act, t, h, a.heads);
 }
 
@@ -487,7 +484,15 @@ __device__ __forceinline__ void attend_one(const Attention& a, const AttLds& l, 
 __global__ __launch_bounds__(256) void k_attention(Attention a) {
     extern __shared__ float4 lds4[];
     const uint32_t t = blockIdx.x / a.heads;
-    attend_one<128>(a, att_lds(reinterpret_cast<float*>(lds4), a.width, a.capacity), t, blockIdx.x - t * a.heads);
+    attend_one(a, att_lds(reinterpret_cast<float*>(lds4), a.width, a.capacity), t, blockIdx.x - t * a.heads);
+}
+
+// Whether token t's table entry names positions the cache holds, of the
+// cache row and the length that token `first`'s names.
+__device__ __forceinline__ bool entry_alike(const Attention& a, uint32_t t, uint32_t first) {
+    const int32_t row = a.table[3u * t], last = a.table[3u * t + 1u], length = a.table[3u * t + 2u];
+    return row == a.table[3u * first] && length == a.table[3u * first + 2u] && row >= 0 &&
+           row < (int32_t)a.cache_rows && length > 0 && length <= (int32_t)a.capacity && last >= 0 && last < length;
 }
 
 // The LDS float offset of key float f (position · width + column) of a chunk.
@@ -549,8 +554,9 @@ __device__ __forceinline__ uint32_t stage_keys(const float* kb, uint32_t width, 
 // is -inf (its exponential then +0, which leaves the total as it is) and its
 // value finite (its product then a zero, which leaves the sum as it is): each
 // tile checks the masked keys and values it would leave out (finite, and no
-// dot product able to overflow) and otherwise attends query by query as
-// k_attention does.
+// dot product able to overflow) and otherwise attends query by query with
+// k_attention_rows' steps, as does a tile whose tokens differ in cache row or
+// length or are out of range.
 
 // Query rows of a tile, at most; a workgroup's LDS at most (one workgroup of
 // eight waves a compute unit: two a SIMD, which the vector unit needs to issue
@@ -837,14 +843,6 @@ __device__ __forceinline__ void tile_values(const Attention& a, const TilePass& 
     }
 }
 
-// Whether token t's table entry names positions the cache holds, of the
-// cache row and the length that token `first`'s names.
-__device__ __forceinline__ bool entry_alike(const Attention& a, uint32_t t, uint32_t first) {
-    const int32_t row = a.table[3u * t], last = a.table[3u * t + 1u], length = a.table[3u * t + 2u];
-    return row == a.table[3u * first] && length == a.table[3u * first + 2u] && row >= 0 &&
-           row < (int32_t)a.cache_rows && length > 0 && length <= (int32_t)a.capacity && last >= 0 && last < length;
-}
-
 // The largest magnitudes' bits (a NaN's are above an infinity's) of `count`
 // floats at k and at v (a multiple of 4, 16-byte pieces), thread by thread.
 __device__ __forceinline__ void largest_bits(const float* __restrict__ k, const float* __restrict__ v, uint32_t count,
@@ -876,20 +874,20 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t m) {
     return m;
 }
 
-// The attention of tokens [t0, t0 + count) (a tile of T), head h; false where a
-// masked key or value could reach the host's results, and nothing is written.
-// A tile whose tokens do not share a cache row and length (or hold an entry
-// out of range) is left alone. lds_floats: room for the scores.
+// The attention of tokens [t0, t0 + count) (a tile of T), head h; false, with
+// nothing written, where the tokens do not share a cache row and length (or hold
+// an entry out of range), or a masked key or value could reach the host's
+// results. lds_floats: room for the scores.
 template <int W>
-__device__ __forceinline__ bool attend_tile(const Attention& a, float* lds, uint32_t lds_floats, uint32_t tokens,
-                                            uint32_t T, uint32_t t0, uint32_t count, uint32_t h) {
+__device__ __forceinline__ bool attend_tile(const Attention& a, float* lds, uint32_t lds_floats, uint32_t T,
+                                            uint32_t t0, uint32_t count, uint32_t h, uint32_t tokens) {
     __shared__ uint32_t found[TILE_WAVES][3];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // lane l: the entry of the tile's token l
     const uint32_t mine = t0 + min(lane, count - 1u);
     const int32_t row = a.table[3u * mine], last = a.table[3u * mine + 1u], length = a.table[3u * mine + 2u];
     const int32_t row0 = __builtin_amdgcn_readfirstlane(row), held = __builtin_amdgcn_readfirstlane(length);
-    if (__builtin_amdgcn_ballot_w64(!entry_alike(a, mine, t0)) != 0) return true;
+    if (__builtin_amdgcn_ballot_w64(!entry_alike(a, mine, t0)) != 0) return false;
     const uint32_t kv = h / (a.heads / a.kv_heads);
     const size_t base = ((size_t)row0 * a.kv_heads + kv) * a.capacity * W;
     const float* kb = a.keys + base;
@@ -986,53 +984,6 @@ __device__ __forceinline__ bool attend_tile(const Attention& a, float* lds, uint
     return true;
 }
 
-// Workgroups [0, tiles · heads): a tile of T tokens (8, 16 or 32)
-// and a head; those after them attend the tokens of tiles that name more than
-// one cache row or length one by one.
-template <int W>
-__global__ __launch_bounds__(TILE_THREADS, 2) void k_attention_tile(Attention a, uint32_t tokens, uint32_t T, uint32_t tiles,
-                                                           uint32_t lds_floats) {
-    extern __shared__ float4 lds4[];
-    __shared__ uint32_t ragged;
-    float* lds = reinterpret_cast<float*>(lds4);
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, work = tiles * a.heads;
-    // query rows to attend one by one: every `step` from item to items (token
-    // item / heads, head item % heads)
-    uint32_t item, items, step;
-    const bool others = blockIdx.x >= work;
-    if (others) {
-        if (tid == 0) ragged = 0;
-        __syncthreads();
-        bool other = false;
-        for (uint32_t t = tid; t < tokens; t += TILE_THREADS) other = other || !entry_alike(a, t, t - t % T);
-        if (other) ragged = 1;
-        __syncthreads();
-        if (!ragged) return;
-        item = blockIdx.x - work;
-        items = tokens * a.heads;
-        step = gridDim.x - work;
-    } else {
-        const uint32_t h = blockIdx.x % a.heads, order = blockIdx.x / a.heads;
-        // a prompt's last tiles see most: they go first
-        const uint32_t t0 = (tiles - 1u - order) * T, count = min(T, tokens - t0);
-        if (attend_tile<W>(a, lds, lds_floats, tokens, T, t0, count, h)) return;
-        item = t0 * a.heads + h;
-        items = (t0 + count) * a.heads;
-        step = a.heads;
-    }
-    if (tid >= 256u) return;  // attend_one's threads
-    const AttLds l = att_lds(lds, W, a.capacity);
-    for (; item < items; item += step) {
-        const uint32_t t = item / a.heads, h = item - t * a.heads, first = t - t % T;
-        const uint32_t other = first + (lane < T ? lane : 0u);
-        // the workgroups after the tiles: tokens of whole tiles are not theirs
-        // (the same answer in every wave)
-        if (others && __builtin_amdgcn_ballot_w64(other < tokens && !entry_alike(a, other, first)) == 0) continue;
-        attend_one<32>(a, l, t, h);
-        __syncthreads();
-    }
-}
-
 // ------------------------------------------------------- few query rows
 //
 // One query row and head a workgroup of eight waves, for launches of at most
@@ -1085,14 +1036,12 @@ __device__ __forceinline__ void add_key_columns(float& dot, const float (&x)[W /
 // are rotated here from the qkv row, and the group's first head writes the new
 // key and value into the caches, which the others do not read there.
 template <int W, bool EARLY, bool ROPE>
-__global__ __launch_bounds__(ROWS_THREADS, 2) void k_attention_rows(Attention a, RopeWrite r, uint32_t kwaves) {
-    extern __shared__ float4 lds4[];
+__device__ __forceinline__ void attend_rows(const Attention& a, const RopeWrite& r, float* lds, uint32_t kwaves,
+                                            uint32_t t, uint32_t h) {
     __shared__ float tops[ROWS_WAVES];
     __shared__ float total_slot, first_slot;
     constexpr uint32_t P = 4096u / W, C = W / 64;  // positions of a block; a lane's columns
-    float* lds = reinterpret_cast<float*>(lds4);
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t t = blockIdx.x / a.heads, h = blockIdx.x - t * a.heads;
     const int32_t row = a.table[3u * t], last = a.table[3u * t + 1u], length = a.table[3u * t + 2u];
     float* out = a.dst + (size_t)t * a.ld_dst + (size_t)h * W;
     const int32_t slot = ROPE ? r.slots[t] : 0, cap = (int32_t)a.capacity;
@@ -1320,6 +1269,33 @@ __global__ __launch_bounds__(ROWS_THREADS, 2) void k_attention_rows(Attention a,
     emit(sums, out, W, a.act, t, h, a.heads);
 }
 
+template <int W, bool EARLY, bool ROPE>
+__global__ __launch_bounds__(ROWS_THREADS, 2) void k_attention_rows(Attention a, RopeWrite r, uint32_t kwaves) {
+    extern __shared__ float4 lds4[];
+    const uint32_t t = blockIdx.x / a.heads;
+    attend_rows<W, EARLY, ROPE>(a, r, reinterpret_cast<float*>(lds4), kwaves, t, blockIdx.x - t * a.heads);
+}
+
+// The prompt kernel. Workgroup: a tile of T tokens (8, 16 or 32) and a head. A
+// tile that names more than one cache row or length, or whose masked positions
+// take part, goes query row by query row. lds_floats: the scores' room; kwaves:
+// attend_rows'.
+template <int W>
+__global__ __launch_bounds__(TILE_THREADS, 2) void k_attention_tile(Attention a, uint32_t tokens, uint32_t T, uint32_t tiles,
+                                                                    uint32_t lds_floats, uint32_t kwaves) {
+    static_assert(TILE_THREADS == ROWS_THREADS, "one workgroup runs both");
+    extern __shared__ float4 lds4[];
+    float* lds = reinterpret_cast<float*>(lds4);
+    const uint32_t h = blockIdx.x % a.heads, order = blockIdx.x / a.heads;
+    // a prompt's last tiles see most: they go first
+    const uint32_t t0 = (tiles - 1u - order) * T, count = min(T, tokens - t0);
+    if (attend_tile<W>(a, lds, lds_floats, T, t0, count, h, tokens)) return;
+    for (uint32_t t = t0; t < t0 + count; ++t) {
+        attend_rows<W, false, false>(a, RopeWrite{}, lds, kwaves, t, h);
+        __syncthreads();
+    }
+}
+
 // Head widths 64 and 128, at most a workgroup a compute unit (each takes its
 // LDS), and caches aligned for the keys' direct loads of 16 bytes.
 static bool rows_fits(const Attention& a, uint32_t tokens, int compute_units) {
@@ -1327,11 +1303,16 @@ static bool rows_fits(const Attention& a, uint32_t tokens, int compute_units) {
            (uint64_t)tokens * a.heads <= (uint64_t)compute_units;
 }
 
+// The waves for whose key blocks a workgroup's LDS has room.
+static uint32_t rows_kwaves(const Attention& a, size_t lds) {
+    const size_t fixed = rows_fixed_floats(a.width, a.capacity) * sizeof(float), block = ROWS_KEY_FLOATS * sizeof(float);
+    return lds < fixed ? 0u : (uint32_t)std::min<size_t>(ROWS_WAVES, (lds - fixed) / block);
+}
+
 template <bool ROPE>
 static hipError_t launch_rows(const Attention& a, const RopeWrite& r, uint32_t tokens, hipStream_t stream) {
-    const size_t fixed = rows_fixed_floats(a.width, a.capacity) * sizeof(float), block = ROWS_KEY_FLOATS * sizeof(float);
-    const uint32_t kwaves = (uint32_t)std::min<size_t>(ROWS_WAVES, (ROWS_LDS - fixed) / block);
-    const size_t lds = fixed + kwaves * block;
+    const uint32_t kwaves = rows_kwaves(a, ROWS_LDS);
+    const size_t lds = (rows_fixed_floats(a.width, a.capacity) + kwaves * ROWS_KEY_FLOATS) * sizeof(float);
     const dim3 grid(tokens * a.heads), threads(ROWS_THREADS);
     const bool early = a.capacity <= 2048u;
     if (a.width == 64u && early)
@@ -1346,20 +1327,21 @@ static hipError_t launch_rows(const Attention& a, const RopeWrite& r, uint32_t t
 }
 
 // Fewest tokens the tiles take (a decode step's sequences are fewer, each with
-// a cache row of its own), and workgroups of k_attention a compute unit holds
-// at a time: up to one such round the tiles gain little and their longer
-// start costs (9 heads of 64, no past: 64 tokens 8.6 us against 9.2 in tiles,
-// 100 tokens 15.8 against 10.0; 32 heads: 16 tokens 6.9 against 7.7, 32 tokens
-// 11.7 against 8.3, 128 tokens 49 against 20, 512 tokens 469 against 65).
-// The tiles' 16-byte loads need the caches 16-byte aligned.
-constexpr uint32_t TILE_MIN_TOKENS = 16, ROUND_WGS = 3;
+// a cache row of its own). Where k_attention's workgroups, of which a compute
+// unit holds three, are fewer than 2.5 a compute unit, the tiles gain little
+// and their longer start costs (9 heads of 64, no past: 64 tokens 8.6 us against
+// 9.2 in tiles, 77 tokens 11.6 against 9.6, 100 tokens 15.8 against 10.0; 32
+// heads: 16 tokens 6.9 against 7.7, 32 tokens 11.7 against 8.3, 128 tokens 49
+// against 20, 512 tokens 469 against 65). The tiles' 16-byte loads need the
+// caches 16-byte aligned.
+constexpr uint32_t TILE_MIN_TOKENS = 16;
 
-hipError_t launch_attention(const Attention& a, uint32_t tokens, bool prompt, int compute_units, hipStream_t stream) {
+hipError_t launch_attention(const Attention& a, uint32_t tokens, int compute_units, hipStream_t stream) {
     if (tokens == 0 || a.heads == 0) return hipSuccess;
     const size_t lds = attention_lds(a.width, a.capacity);
     const bool aligned = (((uintptr_t)a.keys | (uintptr_t)a.values) & 15u) == 0;
     if (rows_fits(a, tokens, compute_units)) return launch_rows<false>(a, RopeWrite{}, tokens, stream);
-    if (tokens < TILE_MIN_TOKENS || (uint64_t)tokens * a.heads < ROUND_WGS * (uint64_t)compute_units ||
+    if (tokens < TILE_MIN_TOKENS || 2u * (uint64_t)tokens * a.heads < 5u * (uint64_t)compute_units ||
         (a.width != 64u && a.width != 128u) || !aligned) {
         TMH_LAUNCH(k_attention, dim3(tokens * a.heads), dim3(256), lds, stream, a);
         return hipGetLastError();
@@ -1372,17 +1354,18 @@ hipError_t launch_attention(const Attention& a, uint32_t tokens, bool prompt, in
     const uint32_t tiles = (tokens + T - 1u) / T, work = tiles * a.heads;
     const size_t row = a.width == 64u ? tile_row_floats<64>(a.capacity) : tile_row_floats<128>(a.capacity);
     const size_t fixed = tile_fixed_floats(a.width, T);
-    const size_t tile_lds = std::max(lds, std::min(TILE_LDS, (fixed + T * row) * sizeof(float)));
-    if ((fixed + 8u * row) * sizeof(float) > tile_lds) {  // no room for eight queries' scores
+    const size_t tile_lds = std::min(TILE_LDS, (fixed + T * row) * sizeof(float));
+    // room for eight queries' scores, and for a query row by itself
+    if ((fixed + 8u * row) * sizeof(float) > tile_lds || rows_kwaves(a, tile_lds) == 0) {
         TMH_LAUNCH(k_attention, dim3(tokens * a.heads), dim3(256), lds, stream, a);
         return hipGetLastError();
     }
-    const uint32_t others = prompt ? 0u : std::min(tokens * a.heads, full);
     const uint32_t floats = (uint32_t)(tile_lds / sizeof(float));
+    const uint32_t kwaves = rows_kwaves(a, tile_lds);
     if (a.width == 64u)
-        TMH_LAUNCH(k_attention_tile<64>, dim3(work + others), dim3(TILE_THREADS), tile_lds, stream, a, tokens, T, tiles, floats);
+        TMH_LAUNCH(k_attention_tile<64>, dim3(work), dim3(TILE_THREADS), tile_lds, stream, a, tokens, T, tiles, floats, kwaves);
     else
-        TMH_LAUNCH(k_attention_tile<128>, dim3(work + others), dim3(TILE_THREADS), tile_lds, stream, a, tokens, T, tiles, floats);
+        TMH_LAUNCH(k_attention_tile<128>, dim3(work), dim3(TILE_THREADS), tile_lds, stream, a, tokens, T, tiles, floats, kwaves);
     return hipGetLastError();
 }
 

@@ -334,12 +334,11 @@ __device__ __forceinline__ float ordered_sum_by_wave(const float* v, uint32_t n)
 }
 
 // The ordered sum of v[0..n) by wave 0 (ordered_sum_by_wave; beyond its
-// limit, ordered_sum), shared through LDS. Every thread calls it. MAXM as there.
-template <int MAXM = 128>
+// limit, ordered_sum), shared through LDS. Every thread calls it.
 __device__ __forceinline__ float shared_sum(const float* v, uint32_t n) {
     __shared__ float result;
     if (threadIdx.x < 64u) {
-        const float sum = n <= 64u * MAXM ? ordered_sum_by_wave<false, MAXM>(v, n) : ordered_sum(v, n);
+        const float sum = n <= WAVE_SUM_MAX ? ordered_sum_by_wave(v, n) : ordered_sum(v, n);
         if (threadIdx.x == 0) result = sum;
     }
     __syncthreads();
@@ -419,6 +418,23 @@ __device__ __forceinline__ void rmsnorm_quantise_row(const float* __restrict__ x
             ((int32_t*)act.totals)[g] = q.total;
         }
     }
+}
+
+// ------------------------------------------------------------------- bias
+
+// v[i] + bias of output (row + i, col) for i < N, bias rows ld floats apart (0:
+// one row for all), as the host adds it: a rounding of its own. Before any
+// store of the outputs: a wait for a load at each store would wait for the
+// store before it as well.
+template <int N, typename V>
+__device__ __forceinline__ void add_bias(V&& v, const float* __restrict__ bias, uint32_t ld, uint32_t row,
+                                         uint32_t col, uint32_t m, uint32_t n) {
+    if (!bias) return;
+    float b[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) b[i] = bias[(size_t)min(row + i, m - 1u) * ld + min(col, n - 1u)];
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = v[i] + b[i];
 }
 
 // ------------------------------------------------- LDS direct loads (gfx950)

@@ -59,7 +59,8 @@ hipError_t launch_quantize(const float* x, uint32_t ldx, uint32_t rows, uint32_t
 enum MxTile { MX_32X32, MX_64X64, MX_64X128, MX_128X128 };
 MxTile mx_tile(uint32_t rows, uint32_t n, int compute_units);
 hipError_t launch_matmul_tiles(uint32_t kind, MxTile tile, const uint8_t* w, Activations act, float* dst,
-                               const float* bias, uint32_t rows, uint32_t n, uint32_t k, hipStream_t stream);
+                               const float* bias, uint32_t bias_ld, uint32_t rows, uint32_t n, uint32_t k,
+                               hipStream_t stream);
 
 // Launches dst[rows, n] = x · wᵀ (+ bias) over quantised activations, in the
 // kernel `mode` asks for (TMH_MODE_*). `w` points at the first weight row.
@@ -178,9 +179,8 @@ hipError_t make_stream(uint32_t kind, std::vector<StreamProduct>& products, int 
 // Launches the streamed one-row kernel (table and starts in device memory).
 hipError_t launch_stream(uint32_t kind, const StreamLaunch& launch, hipStream_t stream);
 
-// dst[rows, n] = residual[rows, n] + act · wᵀ for a few activation rows
-// (fewer than the matrix cores take), the residual added in the product's
-// fold as a bias row per activation row: the host's `x + product`, one
+// dst[rows, n] = residual[rows, n] + act · wᵀ, the residual added after the
+// product's fold as a bias row per activation row: the host's `x + product`, one
 // rounding. hipErrorInvalidValue when the shape is not for that kernel.
 hipError_t launch_product_residual(uint32_t kind, const uint8_t* w, Activations act, float* dst, const float* residual,
                                    uint32_t rows, uint32_t n, uint32_t k, int compute_units, hipStream_t stream);
@@ -297,8 +297,7 @@ struct Attention {
 };
 size_t attention_lds(uint32_t width, uint32_t capacity);
 size_t attention_decode_lds(uint32_t width, uint32_t capacity);  // of launch_attention_decode
-// `prompt`: every token is known to name the same cache row and length, in range.
-hipError_t launch_attention(const Attention& a, uint32_t tokens, bool prompt, int compute_units, hipStream_t stream);
+hipError_t launch_attention(const Attention& a, uint32_t tokens, int compute_units, hipStream_t stream);
 // A decode step's attention with the RoPE and cache write of `r` fused: each
 // token is its cache row's one new position.
 hipError_t launch_attention_decode(const Attention& a, const RopeWrite& r, uint32_t tokens, int compute_units,

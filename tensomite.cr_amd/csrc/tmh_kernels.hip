@@ -1605,7 +1605,7 @@ __device__ __forceinline__ void stage_store(MmStage& S, const MmLoad<KIND>& L) {
 template <int KIND>
 __global__ __launch_bounds__(256) void k_matmul_mfma(const uint8_t* __restrict__ w, Activations act,
                                                      float* __restrict__ dst, const float* __restrict__ bias,
-                                                     uint32_t m, uint32_t n, uint32_t k) {
+                                                     uint32_t m, uint32_t n, uint32_t k, uint32_t bias_ld) {
     __shared__ MmStage stage[2];
     const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
     const uint32_t nb = k >> 5, pairs = nb >> 1;
@@ -1701,12 +1701,17 @@ __global__ __launch_bounds__(256) void k_matmul_mfma(const uint8_t* __restrict__
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
+        for (int b = 0; b < 2; ++b)
+            add_bias<4>(acc[a][b], bias, bias_ld, m0 + wm0 + 16u * a + 4u * lq, n0 + wn0 + 16u * b + lr, m, n);
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
         for (int b = 0; b < 2; ++b) {
             const uint32_t col = n0 + wn0 + 16u * b + lr;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const uint32_t row = m0 + wm0 + 16u * a + 4u * lq + i;
-                if (row < m && col < n) dst[(size_t)row * n + col] = bias ? acc[a][b][i] + bias[col] : acc[a][b][i];
+                if (row < m && col < n) dst[(size_t)row * n + col] = acc[a][b][i];
             }
         }
 }
@@ -1943,7 +1948,7 @@ __device__ __forceinline__ void mx_add(float (&acc)[16], const MxBlock& o) {
 template <int KIND, bool FUSED>
 __global__ __launch_bounds__(MX_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_matmul_mx(
     const uint8_t* __restrict__ w, Activations act, float* __restrict__ dst, const float* __restrict__ bias,
-    uint32_t m, uint32_t n, uint32_t k, uint32_t tiles_m, uint32_t tiles) {
+    uint32_t m, uint32_t n, uint32_t k, uint32_t tiles_m, uint32_t tiles, uint32_t bias_ld) {
     using M = Mx<KIND>;
     __shared__ __attribute__((aligned(16))) uint8_t lds[M::LDS];
     const uint32_t t = threadIdx.x, lane = t & 63u;
@@ -2084,12 +2089,12 @@ __global__ __launch_bounds__(MX_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
 
     if (producer) return;
     const uint32_t col = n0 + nw + l32;
-    float b = (bias && col < n) ? bias[col] : 0.0f;
-    asm volatile("" : "+v"(b));  // waited for here, once: not before every store, with the stores before it
+#pragma unroll
+    for (int i = 0; i < 16; i += 4) add_bias<4>(acc + i, bias, bias_ld, m0 + mw + 2u * i + 4u * half, col, m, n);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         const uint32_t row = m0 + mw + 8u * (i / 4) + 4u * half + (i % 4);
-        if (row < m && col < n) dst[(size_t)row * n + col] = bias ? acc[i] + b : acc[i];
+        if (row < m && col < n) dst[(size_t)row * n + col] = acc[i];
     }
 }
 
@@ -3549,10 +3554,10 @@ hipError_t launch_stream(uint32_t kind, const StreamLaunch& given, hipStream_t s
 }
 
 template <int KIND>
-static hipError_t launch_mfma(const uint8_t* w, Activations act, float* dst, const float* bias, uint32_t rows,
-                              uint32_t n, uint32_t k, hipStream_t stream) {
+static hipError_t launch_mfma(const uint8_t* w, Activations act, float* dst, const float* bias, uint32_t bias_ld,
+                              uint32_t rows, uint32_t n, uint32_t k, hipStream_t stream) {
     const dim3 grid((n + MM_TILE - 1u) / MM_TILE, (rows + MM_TILE - 1u) / MM_TILE);
-    TMH_LAUNCH(k_matmul_mfma<KIND>, grid, dim3(256), 0, stream, w, act, dst, bias, rows, n, k);
+    TMH_LAUNCH(k_matmul_mfma<KIND>, grid, dim3(256), 0, stream, w, act, dst, bias, rows, n, k, bias_ld);
     return hipGetLastError();
 }
 
@@ -3568,14 +3573,14 @@ static bool mx_fits(const uint8_t* w, const Activations& act, uint32_t kind, uin
 
 template <int KIND>
 static hipError_t launch_mx(bool fused, const uint8_t* w, Activations act, float* dst, const float* bias,
-                            uint32_t rows, uint32_t n, uint32_t k, hipStream_t stream) {
+                            uint32_t bias_ld, uint32_t rows, uint32_t n, uint32_t k, hipStream_t stream) {
     const uint32_t tiles_m = (rows + MX_TILE - 1u) / MX_TILE, tiles = tiles_m * ((n + MX_TILE - 1u) / MX_TILE);
     if (fused)
         TMH_LAUNCH((k_matmul_mx<KIND, true>), dim3(tiles), dim3(MX_THREADS), 0, stream, w, act, dst, bias,
-                           rows, n, k, tiles_m, tiles);
+                           rows, n, k, tiles_m, tiles, bias_ld);
     else
         TMH_LAUNCH((k_matmul_mx<KIND, false>), dim3(tiles), dim3(MX_THREADS), 0, stream, w, act, dst, bias,
-                           rows, n, k, tiles_m, tiles);
+                           rows, n, k, tiles_m, tiles, bias_ld);
     return hipGetLastError();
 }
 
@@ -3637,6 +3642,26 @@ static bool few_rows_kernel() {
     return !lanes;
 }
 
+// The matrix-core product, bias rows bias_ld floats apart (0: one row for all).
+static hipError_t launch_matrix(uint32_t kind, bool fused, const uint8_t* w, Activations act, float* dst,
+                                const float* bias, uint32_t bias_ld, uint32_t rows, uint32_t n, uint32_t k,
+                                int compute_units, hipStream_t stream) {
+    if (mx_fits(w, act, kind, k)) {
+        const MxTile tile = fused ? MX_64X64 : mx_tile(rows, n, compute_units);
+        if (tile != MX_64X64) return launch_matmul_tiles(kind, tile, w, act, dst, bias, bias_ld, rows, n, k, stream);
+        switch (kind) {
+        case 0: return launch_mx<0>(fused, w, act, dst, bias, bias_ld, rows, n, k, stream);
+        case 1: return launch_mx<1>(fused, w, act, dst, bias, bias_ld, rows, n, k, stream);
+        default: return launch_mx<2>(fused, w, act, dst, bias, bias_ld, rows, n, k, stream);
+        }
+    }
+    switch (kind) {
+    case 0: return launch_mfma<0>(w, act, dst, bias, bias_ld, rows, n, k, stream);
+    case 1: return launch_mfma<1>(w, act, dst, bias, bias_ld, rows, n, k, stream);
+    default: return launch_mfma<2>(w, act, dst, bias, bias_ld, rows, n, k, stream);
+    }
+}
+
 hipError_t launch_block_matmul(uint32_t kind, uint32_t mode, const uint8_t* w, Activations act, float* dst,
                                const float* bias, uint32_t rows, uint32_t n, uint32_t k, int compute_units,
                                hipStream_t stream) {
@@ -3647,15 +3672,8 @@ hipError_t launch_block_matmul(uint32_t kind, uint32_t mode, const uint8_t* w, A
     // Below MATRIX_ROWS, UNORDERED takes AUTO's kernels, each folding in its
     // own order (tree_fold, set by the entry point)
     const bool autoish = mode == 0u /* AUTO */ || mode == 3u /* UNORDERED */;
-    if ((matrix || fused) && mx_fits(w, act, kind, k)) {
-        const MxTile tile = fused ? MX_64X64 : mx_tile(rows, n, compute_units);
-        if (tile != MX_64X64) return launch_matmul_tiles(kind, tile, w, act, dst, bias, rows, n, k, stream);
-        switch (kind) {
-        case 0: return launch_mx<0>(fused, w, act, dst, bias, rows, n, k, stream);
-        case 1: return launch_mx<1>(fused, w, act, dst, bias, rows, n, k, stream);
-        default: return launch_mx<2>(fused, w, act, dst, bias, rows, n, k, stream);
-        }
-    }
+    if ((matrix || fused) && mx_fits(w, act, kind, k))
+        return launch_matrix(kind, fused, w, act, dst, bias, 0, rows, n, k, compute_units, stream);
     if (autoish && (rows == 1u || rows == 8u) && few_rows_kernel()) {
         // one or 8 rows: the weights of each workgroup's tile staged into LDS
         // at once, the products on the matrix cores (measured, Q4_1: 8 rows
@@ -3669,13 +3687,7 @@ hipError_t launch_block_matmul(uint32_t kind, uint32_t mode, const uint8_t* w, A
     }
     if (autoish && few_fits(w, act, kind, rows, k))
         return launch_few_kind(kind, w, act, dst, bias, 0, rows, n, k, stream);
-    if (matrix) {
-        switch (kind) {
-        case 0: return launch_mfma<0>(w, act, dst, bias, rows, n, k, stream);
-        case 1: return launch_mfma<1>(w, act, dst, bias, rows, n, k, stream);
-        default: return launch_mfma<2>(w, act, dst, bias, rows, n, k, stream);
-        }
-    }
+    if (matrix) return launch_matrix(kind, false, w, act, dst, bias, 0, rows, n, k, compute_units, stream);
     const bool thread = mode == 1u /* THREAD */ || !fits;
     switch (kind) {
     case 0:
@@ -3693,7 +3705,9 @@ hipError_t launch_block_matmul(uint32_t kind, uint32_t mode, const uint8_t* w, A
 hipError_t launch_product_residual(uint32_t kind, const uint8_t* w, Activations act, float* dst, const float* residual,
                                   uint32_t rows, uint32_t n, uint32_t k, int compute_units, hipStream_t stream) {
     if (rows == 0 || n == 0) return hipSuccess;
-    if (!lanes_fit(w, k) || rows >= MATRIX_ROWS) return hipErrorInvalidValue;
+    if (!lanes_fit(w, k)) return hipErrorInvalidValue;
+    if (rows >= MATRIX_ROWS)
+        return launch_matrix(kind, false, w, act, dst, residual, n, rows, n, k, compute_units, stream);
     if (few_fits(w, act, kind, rows, k)) return launch_few_kind(kind, w, act, dst, residual, n, rows, n, k, stream);
     switch (kind) {
     case 0: return launch_lanes<0>(w, act, dst, residual, rows, n, k, compute_units, stream, n);

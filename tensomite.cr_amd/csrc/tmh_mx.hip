@@ -40,7 +40,7 @@ namespace tmh {
 // tile comes from HBM once, into that XCD's L2.
 //
 // Measured (a call, quantise pass included): Q8_0 512 x 2048 -> 8192 60.0 ->
-// 36.1 us, Q4_0 67.0 -> 39.2, Q4_0 100 x 2048 -> 16384 35.0 -> 24.7, 100 x 8192
+// 35.5 us, Q4_0 67.0 -> 39.2, Q4_0 100 x 2048 -> 16384 35.0 -> 24.7, 100 x 8192
 // -> 2048 53.6 -> 34.7.
 constexpr uint32_t MX_STAGE = 8;
 constexpr uint32_t MX_ROW = 272;  // LDS bytes per activation row (256 + a 16-byte pad)
@@ -225,8 +225,8 @@ __device__ __forceinline__ void mx_add(float (&acc)[E], const MxBlock& o, float 
 
 template <int KIND, int MS, int WN, int WM, int FS, int PART>
 __device__ __forceinline__ void mx_product(uint8_t* lds, const uint8_t* __restrict__ w, const Activations& act,
-                                           float* __restrict__ dst, const float* __restrict__ bias, uint32_t m,
-                                           uint32_t n, uint32_t k, uint32_t tiles_m, uint32_t tiles) {
+                                           float* __restrict__ dst, const float* __restrict__ bias,
+                                           uint32_t bias_ld, uint32_t m, uint32_t n, uint32_t k, uint32_t tiles_m, uint32_t tiles) {
     using M = Mx<KIND, MS, WN, WM, FS>;
     constexpr bool PIPE = M::WAVES < 16;  // four waves a SIMD hide an MFMA's latency by themselves
     constexpr bool FACTORS = mx_factors<FS>;
@@ -411,15 +411,18 @@ __device__ __forceinline__ void mx_product(uint8_t* lds, const uint8_t* __restri
 
     const uint32_t col = n0 + 32u * wn + l32;
     if (col >= n) return;
-    float b = bias ? bias[col] : 0.0f;
-    asm volatile("" : "+v"(b));  // waited for here, once: not before every store, with the stores before it
+#pragma unroll
+    for (int i = 0; i < MS; ++i)
+#pragma unroll
+        for (int e = 0; e < E; e += 4)
+            add_bias<4>(acc[i] + e, bias, bias_ld, m0 + (wm * MS + i) * 32u + 2u * (FIRST + e) + 4u * half, col, m, n);
 #pragma unroll
     for (int i = 0; i < MS; ++i)
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const int o = FIRST + e;
             const uint32_t row = m0 + (wm * MS + i) * 32u + 8u * (o / 4) + 4u * half + (o % 4);
-            if (row < m) dst[(size_t)row * n + col] = bias ? acc[i][e] + b : acc[i][e];
+            if (row < m) dst[(size_t)row * n + col] = acc[i][e];
         }
 }
 
@@ -431,17 +434,18 @@ __device__ __forceinline__ void mx_product(uint8_t* lds, const uint8_t* __restri
     __global__ __launch_bounds__(64 * WN * WM * FS)                                                                \
         __attribute__((amdgpu_waves_per_eu(WN * WM * FS / 4, WN * WM * FS / 4))) void NAME(                        \
             const uint8_t* __restrict__ w, Activations act, float* __restrict__ dst,                               \
-            const float* __restrict__ bias, uint32_t m, uint32_t n, uint32_t k, uint32_t tiles_m, uint32_t tiles) { \
+            const float* __restrict__ bias, uint32_t m, uint32_t n, uint32_t k, uint32_t tiles_m, uint32_t tiles,  \
+            uint32_t bias_ld) {                                                                                    \
         __shared__ __attribute__((aligned(16))) uint8_t lds[Mx<KIND, MS, WN, WM, FS>::LDS];                        \
         const uint32_t part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / (WN * WM);                        \
         if (FS == 1 || part == 0)                                                                                  \
-            mx_product<KIND, MS, WN, WM, FS, 0>(lds, w, act, dst, bias, m, n, k, tiles_m, tiles);                  \
+            mx_product<KIND, MS, WN, WM, FS, 0>(lds, w, act, dst, bias, bias_ld, m, n, k, tiles_m, tiles);                  \
         else if (part == 1)                                                                                        \
-            mx_product<KIND, MS, WN, WM, FS, 1 % FS>(lds, w, act, dst, bias, m, n, k, tiles_m, tiles);             \
+            mx_product<KIND, MS, WN, WM, FS, 1 % FS>(lds, w, act, dst, bias, bias_ld, m, n, k, tiles_m, tiles);             \
         else if (part == 2)                                                                                        \
-            mx_product<KIND, MS, WN, WM, FS, 2 % FS>(lds, w, act, dst, bias, m, n, k, tiles_m, tiles);             \
+            mx_product<KIND, MS, WN, WM, FS, 2 % FS>(lds, w, act, dst, bias, bias_ld, m, n, k, tiles_m, tiles);             \
         else                                                                                                       \
-            mx_product<KIND, MS, WN, WM, FS, 3 % FS>(lds, w, act, dst, bias, m, n, k, tiles_m, tiles);             \
+            mx_product<KIND, MS, WN, WM, FS, 3 % FS>(lds, w, act, dst, bias, bias_ld, m, n, k, tiles_m, tiles);             \
     }
 TMH_MX_KERNEL(k_matmul_128x128, 1, 4, 4, 1)  // rows x outputs of a workgroup
 TMH_MX_KERNEL(k_matmul_64x128, 1, 4, 2, 1)
@@ -471,24 +475,28 @@ MxTile mx_tile(uint32_t rows, uint32_t n, int compute_units) {
 
 template <int KIND>
 static hipError_t launch_tiles(MxTile tile, const uint8_t* w, Activations act, float* dst, const float* bias,
-                               uint32_t rows, uint32_t n, uint32_t k, hipStream_t stream) {
+                               uint32_t bias_ld, uint32_t rows, uint32_t n, uint32_t k, hipStream_t stream) {
     const uint32_t tm = tile == MX_128X128 ? 128u : tile == MX_64X128 ? 64u : 32u, tn = tile == MX_32X32 ? 32u : 128u;
     const uint32_t tiles_m = (rows + tm - 1u) / tm, tiles = tiles_m * ((n + tn - 1u) / tn);
     if (tile == MX_128X128)
-        TMH_LAUNCH(k_matmul_128x128<KIND>, dim3(tiles), dim3(1024), 0, stream, w, act, dst, bias, rows, n, k, tiles_m, tiles);
+        TMH_LAUNCH(k_matmul_128x128<KIND>, dim3(tiles), dim3(1024), 0, stream, w, act, dst, bias, rows, n, k, tiles_m,
+                   tiles, bias_ld);
     else if (tile == MX_64X128)
-        TMH_LAUNCH(k_matmul_64x128<KIND>, dim3(tiles), dim3(512), 0, stream, w, act, dst, bias, rows, n, k, tiles_m, tiles);
+        TMH_LAUNCH(k_matmul_64x128<KIND>, dim3(tiles), dim3(512), 0, stream, w, act, dst, bias, rows, n, k, tiles_m,
+                   tiles, bias_ld);
     else
-        TMH_LAUNCH(k_matmul_32x32<KIND>, dim3(tiles), dim3(256), 0, stream, w, act, dst, bias, rows, n, k, tiles_m, tiles);
+        TMH_LAUNCH(k_matmul_32x32<KIND>, dim3(tiles), dim3(256), 0, stream, w, act, dst, bias, rows, n, k, tiles_m,
+                   tiles, bias_ld);
     return hipGetLastError();
 }
 
 hipError_t launch_matmul_tiles(uint32_t kind, MxTile tile, const uint8_t* w, Activations act, float* dst,
-                               const float* bias, uint32_t rows, uint32_t n, uint32_t k, hipStream_t stream) {
+                               const float* bias, uint32_t bias_ld, uint32_t rows, uint32_t n, uint32_t k,
+                               hipStream_t stream) {
     switch (kind) {
-    case 0: return launch_tiles<0>(tile, w, act, dst, bias, rows, n, k, stream);
-    case 1: return launch_tiles<1>(tile, w, act, dst, bias, rows, n, k, stream);
-    default: return launch_tiles<2>(tile, w, act, dst, bias, rows, n, k, stream);
+    case 0: return launch_tiles<0>(tile, w, act, dst, bias, bias_ld, rows, n, k, stream);
+    case 1: return launch_tiles<1>(tile, w, act, dst, bias, bias_ld, rows, n, k, stream);
+    default: return launch_tiles<2>(tile, w, act, dst, bias, bias_ld, rows, n, k, stream);
     }
 }
 

@@ -1,10 +1,11 @@
 """The matrix-core kernels' workgroup tiles (32 x 32, 64 x 64, 64 x 128 and 128 x
 128 rows x outputs) against the oracle, bit for bit: whole and ragged rows and
 outputs, one stage of 8 blocks to more than the ring of buffers holds, a bias,
-a weight row slice, scales that are subnormal or not finite."""
+a weight row slice, scales that are subnormal or not finite, a residual."""
 import numpy as np
 import pytest
 
+from llama_fixtures import random_llama
 from oracle import oracle
 import tensomite_hip as th
 
@@ -68,3 +69,19 @@ def test_scales_not_finite(dev, fmt, shape):
     nan = np.isnan(want)
     assert np.array_equal(np.isnan(got), nan)
     assert np.array_equal(got.view(np.uint32)[~nan], want.view(np.uint32)[~nan])
+
+
+# (width, ids): the residual added in the product, where the 32 x 32 tiles, the
+# 64 x 64 and the 64 x 128 take it, and at a width that none of them takes
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("width,ids", [(256, 32), (256, 45), (576, 33), (1024, 300), (2048, 520)])
+def test_residual_in_the_product(dev, fmt, width, ids):
+    print("residual", fmt, width, ids, flush=True)
+    config = dict(layers=1, width=width, heads=2, kv_heads=1, head_width=64, hidden=352 if width == 576 else 256,
+                  vocab=300, context=ids, eps=1e-5, theta=10000.0, kind=fmt)
+    weights = random_llama(config, seed=width + ids, norm_jitter=0.1)
+    prompt = list(np.random.default_rng(ids).integers(0, config["vocab"], ids))
+    got = th.HIPLlama(dev, config, weights, rows=1, capacity=ids, max_tokens=ids).forward(prompt, last_only=False)
+    want = oracle.Llama(config, weights).forward(prompt, last_only=False)
+    got, want = np.asarray(got, np.float32).reshape(ids, -1), np.asarray(want, np.float32).reshape(ids, -1)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
