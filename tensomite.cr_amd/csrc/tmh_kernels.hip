@@ -2108,11 +2108,17 @@ __global__ __launch_bounds__(MX_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
 // operations a row and block for the dot products).
 //
 // The k axis goes in stages of 16 blocks through a ring of DEPTH LDS
-// buffers, the loads of stages s + 1 .. s + DEPTH - 1 in flight while stage
-// s is computed, one workgroup barrier a stage; all of it by direct loads
-// (raw weight rows, the activation rows 528 bytes apart, their scales and
-// extras). In a stage, wave v issues the v_mfma_i32_16x16x32_i8 of blocks
-// 2v and 2v + 1 (the 16 x 16 tile of rows x outputs of one block; operands
+// buffers (or of 32, launch_few), the loads of stages s + 1 .. s + DEPTH - 1
+// in flight while stage s is computed, one workgroup barrier a stage; all of it
+// by direct loads (raw weight rows, activation rows, their scales and extras).
+// What bounds a stage is its chain of latencies and the LDS: each operand is
+// read from there once, so rows lie an odd number of 16-byte pieces apart and
+// every four rows' scales are followed by a piece of padding, which keeps the
+// 16 rows' (and four lane groups') reads on distinct banks (measured, 16 rows, a
+// call: Q4_1 8192 -> 2048 17.8 -> 16.1 us, 2048 -> 8192 10.0 -> 8.95; Q8_0 8192 ->
+// 2048 18.0 -> 16.7; four more waves for the fold gained nothing on top).
+// In a stage, wave v issues the v_mfma_i32_16x16x32_i8 of its two (or four)
+// blocks (the 16 x 16 tile of rows x outputs of one block; operands
 // read where the blocks lie: Q8_0 values
 // funnel-shifted in even blocks, Q4 nibbles unpacked a dword at a time with
 // the activations taken in the same order; Q4_0's -8·Σq as the MFMA's C),
@@ -2186,14 +2192,16 @@ struct Few {
     static constexpr uint32_t BB = Fmt<KIND>::BB;
     static constexpr uint32_t RB = SB * BB;  // a weight row's bytes in a stage
     static constexpr uint32_t RC = RB / 16u;
+    static constexpr uint32_t WCH = RC | 1u, WROW = 16u * WCH;  // LDS pieces (odd) and bytes per weight row
     static constexpr uint32_t KB1 = 1024u;
-    static constexpr uint32_t W_BYTES = (FEW_COLS * RB + KB1 - 1u) / KB1 * KB1;  // whole 1 KB wave loads
-    static constexpr uint32_t A_CHUNKS = FEW_ROWS * ACH;
-    static constexpr uint32_t A_BYTES = (FEW_ROWS * AROW + KB1 - 1u) / KB1 * KB1;
-    static constexpr uint32_t S_BYTES = FEW_ROWS * SB * 4u;  // scales [row][SB]
+    static constexpr uint32_t W_BYTES = FEW_COLS * WROW;
+    static constexpr uint32_t A_BYTES = FEW_ROWS * AROW;
+    static constexpr uint32_t SCH = SB + 1u, SQUAD = 16u * SCH;  // pieces and bytes per four rows' scales
+    static constexpr uint32_t S_BYTES = FEW_ROWS / 4u * SQUAD;   // scales [row][SB], four rows and a pad
     static constexpr uint32_t E_BYTES = KIND == 0 ? 0u : S_BYTES;  // Q4_0 Σq, Q4_1 sums
     // a raw stage: weights, activations, scales, extras
-    static constexpr uint32_t R_A = W_BYTES, R_S = R_A + A_BYTES, R_E = R_S + S_BYTES, R_BYTES = R_E + E_BYTES;
+    static constexpr uint32_t R_A = W_BYTES, R_S = R_A + A_BYTES, R_E = R_S + S_BYTES;
+    static constexpr uint32_t R_BYTES = (R_E + E_BYTES + KB1 - 1u) / KB1 * KB1;  // whole 1 KB wave loads
     static constexpr uint32_t LOADS = R_BYTES / KB1;
     // a stage's contributions [block][row][output], f32
     static constexpr uint32_t P_BYTES = SB * FEW_ROWS * FEW_COLS * 4u;
@@ -2233,20 +2241,22 @@ __global__ __launch_bounds__(FEW_THREADS) void k_matmul_few(const uint8_t* __res
         if (i >= F::LOADS) continue;
         ++mine;
         if (at < F::R_A) {
-            const uint32_t p = min(at / 16u, FEW_COLS * F::RC - 1u), col = p / F::RC, chunk = p % F::RC;
+            const uint32_t p = at / 16u, col = p / F::WCH;
+            const uint32_t chunk = min(p % F::WCH, F::RC - 1u);
             src[j] = w + (size_t)min(n0 + col, n - 1u) * row_bytes + 16u * chunk;
             step[j] = F::RB;
         } else if (at < F::R_S) {
-            const uint32_t p = min((at - F::R_A) / 16u, F::A_CHUNKS - 1u), row = p / F::ACH;
+            const uint32_t p = (at - F::R_A) / 16u, row = p / F::ACH;
             const uint32_t chunk = min(p % F::ACH, F::ACH - 2u);
             src[j] = (const uint8_t*)act.qs + (size_t)min(row, rows - 1u) * k + 16u * chunk;
             step[j] = SB * 32u;
         } else {
-            const bool ex = at >= F::R_E;
-            const uint32_t p = (at - (ex ? F::R_E : F::R_S)) / 16u, row = p / (SB / 4u);
+            const bool ex = KIND != 0 && at >= F::R_E;
+            const uint32_t p = (at - (ex ? F::R_E : F::R_S)) / 16u, piece = min(p % F::SCH, SB - 1u);
+            const uint32_t row = 4u * (p / F::SCH) + piece / (SB / 4u);
             const void* from = !ex ? (const void*)act.scales
                                    : (KIND == 1 ? (const void*)act.totals : (const void*)act.sums);
-            src[j] = (const uint8_t*)from + ((size_t)min(row, rows - 1u) * nb + 4u * (p % (SB / 4u))) * 4u;
+            src[j] = (const uint8_t*)from + ((size_t)min(row, rows - 1u) * nb + 4u * (piece % (SB / 4u))) * 4u;
             step[j] = SB * 4u;
         }
     }
@@ -2273,12 +2283,12 @@ __global__ __launch_bounds__(FEW_THREADS) void k_matmul_few(const uint8_t* __res
     for (uint32_t s = 0; s <= stages; ++s) {
         if (s + F::NBUF - 1u < stages) issue(s + F::NBUF - 1u);
         if (s < stages) {
-            // This wave's blocks of stage s (2v, 2v + 1): their
+            // This wave's blocks of stage s (PER from PER·v): their
             // contributions, written as the MFMA result lies (block, lane,
             // the lane's 4 rows), one 16-byte write a block.
             const uint8_t* raw = lds + F::RAW + (s % F::NBUF) * F::R_BYTES;
             uint8_t* pk = lds + F::PK + (s & 1u) * F::P_BYTES;
-            const uint8_t* wrow = raw + lr * F::RB;
+            const uint8_t* wrow = raw + lr * F::WROW;
             const uint8_t* arow = raw + F::R_A + lr * F::AROW;
             // the lane's 4 rows' scales (and extras) of the wave's blocks
             float sxv[4][PER], exv[4][PER];
@@ -2286,7 +2296,7 @@ __global__ __launch_bounds__(FEW_THREADS) void k_matmul_few(const uint8_t* __res
             for (int i = 0; i < 4; ++i)
 #pragma unroll
                 for (uint32_t u = 0; u < PER; u += 2u) {
-                    const uint32_t at = ((4u * lq + i) * SB + PER * wave + u) * 4u;
+                    const uint32_t at = lq * F::SQUAD + (i * SB + PER * wave + u) * 4u;
                     const float2 x = *(const float2*)(raw + F::R_S + at);
                     sxv[i][u] = x.x, sxv[i][u + 1u] = x.y;
                     if constexpr (KIND != 0) {
@@ -3602,12 +3612,24 @@ static bool few_fits(const uint8_t* w, const Activations& act, uint32_t kind, ui
 }
 
 // A ring of 3 stage buffers leaves LDS for two workgroups a compute unit
-// (wide products: more than 256 workgroups); narrow ones take a ring of 6.
+// (wide products: more than 256 workgroups; Q4_0 and Q4_1). Narrow ones have a
+// compute unit to themselves: stages of 32 blocks in a ring of 3 where the two
+// Q4 formats' rows are whole such stages (Q8_0's do not fit; a stage's time is
+// mostly its latencies and its barrier: 16 x 8192 -> 2048 Q4_1 16.1 us a call
+// with stages of 16, 13.9 with 32; 12 x 2048 -> 2048 Q4_0 8.1 with either), else
+// stages of 16 in a ring of 6. UNORDERED's sums go by stages of 16 always.
 template <int KIND>
 static hipError_t launch_few(const uint8_t* w, Activations act, float* dst, const float* bias, uint32_t bias_ld,
                              uint32_t rows, uint32_t n, uint32_t k, hipStream_t stream) {
     const uint32_t grid = (n + FEW_COLS - 1u) / FEW_COLS;
     const bool tree = tree_fold();
+    if constexpr (KIND != 0) {
+        if (grid <= 256u && !tree && (k >> 5) % 32u == 0) {
+            TMH_LAUNCH((k_matmul_few<KIND, 3, 32, false>), dim3(grid), dim3(FEW_THREADS), 0, stream, w, act, dst,
+                       bias, bias_ld, rows, n, k);
+            return hipGetLastError();
+        }
+    }
     if (grid > 256u && tree)
         TMH_LAUNCH((k_matmul_few<KIND, 3, 16, true>), dim3(grid), dim3(FEW_THREADS), 0, stream, w, act, dst, bias,
                    bias_ld, rows, n, k);
