@@ -1296,17 +1296,21 @@ __global__ __launch_bounds__(TILE_THREADS, 2) void k_attention_tile(Attention a,
     }
 }
 
-// Head widths 64 and 128, at most a workgroup a compute unit (each takes its
-// LDS), and caches aligned for the keys' direct loads of 16 bytes.
-static bool rows_fits(const Attention& a, uint32_t tokens, int compute_units) {
-    return (((uintptr_t)a.keys | (uintptr_t)a.values) & 15u) == 0 && (a.width == 64u || a.width == 128u) &&
-           (uint64_t)tokens * a.heads <= (uint64_t)compute_units;
-}
-
 // The waves for whose key blocks a workgroup's LDS has room.
 static uint32_t rows_kwaves(const Attention& a, size_t lds) {
     const size_t fixed = rows_fixed_floats(a.width, a.capacity) * sizeof(float), block = ROWS_KEY_FLOATS * sizeof(float);
     return lds < fixed ? 0u : (uint32_t)std::min<size_t>(ROWS_WAVES, (lds - fixed) / block);
+}
+
+// Head widths 64 and 128, at most a workgroup a compute unit (each takes its
+// LDS), caches aligned for the keys' direct loads of 16 bytes, and room beside
+// the capacity's scores for two waves' keys (capacities up to 32000). With one
+// wave's, 32768 positions of 32 heads took 1092 us against 969 with k_attention
+// (2584 against 2109 at width 128); with three waves', 24576 of them 493 against
+// 735; past 36000 positions no wave's fit.
+static bool rows_fits(const Attention& a, uint32_t tokens, int compute_units) {
+    return (((uintptr_t)a.keys | (uintptr_t)a.values) & 15u) == 0 && (a.width == 64u || a.width == 128u) &&
+           (uint64_t)tokens * a.heads <= (uint64_t)compute_units && rows_kwaves(a, ROWS_LDS) >= 2u;
 }
 
 template <bool ROPE>

@@ -137,6 +137,21 @@ def test_few_query_rows(dev, width, capacity, lengths):
         same(got, oracle.attention(q, k, v, table, scale))
 
 
+# Capacities whose scores fill the workgroup's LDS: the last one with room for
+# two waves' keys, the first without, the first without room for one's, and the
+# largest the entry point takes.
+@pytest.mark.parametrize("width,capacity", [(64, 32256), (64, 32257), (64, 36353), (64, 39356),
+                                            (128, 32000), (128, 32001), (128, 36097), (128, 38264)])
+def test_capacities_that_fill_lds(dev, width, capacity):
+    print("capacity", width, capacity, flush=True)
+    lengths = [capacity, 700, 1]
+    q, k, v = inputs(capacity, len(lengths), 2, 1, width, capacity, rows=len(lengths))
+    table = [(i, n - 1, n) for i, n in enumerate(lengths)]
+    got, scale = attend(dev, q, k, v, table)
+    dev.sync()
+    same(got, oracle.attention(q, k, v, table, scale))
+
+
 @pytest.mark.parametrize("head_width,capacity", [(64, 1200), (128, 700), (64, 2600)])
 def test_decode_past_several_rounds(dev, head_width, capacity):
     # the decode step's form (RoPE, the cache write and the new position
