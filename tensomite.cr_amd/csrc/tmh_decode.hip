@@ -683,13 +683,16 @@ __device__ __forceinline__ void tile_scores(const TileStage& s, uint32_t wave) {
     }
 }
 
-// Floats of a score row of n positions: whole stages, plus 4 (the totals'
+// Floats of a score row of n positions: whole stages, and a query's W outputs
+// at least (tile_values' quantiser takes them from there), plus 4 (the totals'
 // 16-byte reads of up to 16 rows then fall on distinct banks).
 template <int W>
 __host__ __device__ constexpr uint32_t tile_row_floats(uint32_t n) {
     constexpr uint32_t STAGE = 64u * tile_blocks(W);
-    return (n + STAGE - 1u) / STAGE * STAGE + 4u;
+    const uint32_t stages = (n + STAGE - 1u) / STAGE * STAGE;
+    return (stages > W ? stages : W) + 4u;
 }
+static_assert(tile_row_floats<64>(1) >= 64u && tile_row_floats<128>(1) >= 128u, "a query's outputs in its score row");
 
 // What a tile's pass needs; S floats a score row.
 struct TilePass {

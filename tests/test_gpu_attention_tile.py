@@ -172,3 +172,22 @@ def test_decode_past_several_rounds(dev, head_width, capacity):
             got = model.forward(ids[at:at + 1])
             assert np.array_equal(got.view(np.uint32)[0], want.view(np.uint32)[at]), at
             at += 1
+
+
+# The decoder's prompts: the tiles' outputs quantised for the o product, whose
+# staging takes a score row as wide as a query's outputs although the first tiles'
+# positions are fewer. Tiles of 8, 16 and 32 tokens (one, two and four queries a
+# wave); the last cases' whole cache is shorter than 64 positions.
+@pytest.mark.parametrize("head_width", [64, 128])
+@pytest.mark.parametrize("heads,tokens,capacity", [
+    (16, 40, 256), (32, 64, 256), (32, 65, 256), (16, 200, 200), (32, 250, 256), (64, 250, 250), (32, 20, 20), (64, 60, 60)])
+def test_prompt_tiles_quantised(dev, head_width, heads, tokens, capacity):
+    from llama_fixtures import random_llama
+    print("quantised tiles", head_width, heads, tokens, capacity, flush=True)
+    config = dict(layers=1, width=64, heads=heads, kv_heads=4, head_width=head_width, hidden=32, vocab=96,
+                  context=capacity, eps=1e-5, theta=10000.0, kind="Q8_0")
+    weights = random_llama(config, seed=tokens + heads, std=0.2)
+    ids = np.random.default_rng(tokens).integers(0, 96, tokens).astype(np.int32)
+    want = oracle.Llama(config, weights).forward([int(i) for i in ids])
+    got = th.HIPLlama(dev, config, weights, max_tokens=tokens).forward(ids)
+    same(got, want)
