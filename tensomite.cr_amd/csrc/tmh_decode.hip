@@ -488,11 +488,41 @@ __global__ __launch_bounds__(256) void k_attention(Attention a) {
 }
 
 // Whether token t's table entry names positions the cache holds, of the
-// cache row and the length that token `first`'s names.
+// cache row that token `first`'s names.
 __device__ __forceinline__ bool entry_alike(const Attention& a, uint32_t t, uint32_t first) {
     const int32_t row = a.table[3u * t], last = a.table[3u * t + 1u], length = a.table[3u * t + 2u];
-    return row == a.table[3u * first] && length == a.table[3u * first + 2u] && row >= 0 &&
-           row < (int32_t)a.cache_rows && length > 0 && length <= (int32_t)a.capacity && last >= 0 && last < length;
+    return row == a.table[3u * first] && row >= 0 && row < (int32_t)a.cache_rows && length > 0 &&
+           length <= (int32_t)a.capacity && last >= 0 && last < length;
+}
+
+// Whether the tile of `count` tokens from t0 holds an entry that is not alike
+// (the same answer in every wave).
+__device__ __forceinline__ bool tile_mixed(const Attention& a, uint32_t t0, uint32_t count) {
+    return __builtin_amdgcn_ballot_w64(!entry_alike(a, t0 + min(threadIdx.x & 63u, count - 1u), t0)) != 0;
+}
+
+// The tokens of the prompt kernel's tiles (of T) that are mixed, launched after it
+// where the cache has more rows than one: query rows and heads as in k_attention,
+// one workgroup's after another, in one round of workgroups (three a compute
+// unit). A prompt's find no such tile and end: 3.6 us.
+__global__ __launch_bounds__(256, 3) void k_attention_mixed(Attention a, uint32_t tokens, uint32_t T) {
+    extern __shared__ float4 lds4[];
+    const AttLds l = att_lds(reinterpret_cast<float*>(lds4), a.width, a.capacity);
+    bool first = true;
+    for (uint32_t item = blockIdx.x; item < tokens * a.heads; item += gridDim.x) {
+        const uint32_t t = item / a.heads, t0 = t - t % T;
+        if (!tile_mixed(a, t0, min(T, tokens - t0))) {
+            // (one look at all of them spares a prompt the look at each)
+            bool other = false;
+            for (uint32_t i = threadIdx.x; first && i < tokens; i += 256u) other = other || !entry_alike(a, i, i - i % T);
+            if (first && __syncthreads_or(other) == 0) return;
+            first = false;
+            continue;
+        }
+        first = false;
+        attend_one(a, l, t, item - t * a.heads);
+        __syncthreads();
+    }
 }
 
 // The LDS float offset of key float f (position · width + column) of a chunk.
@@ -555,8 +585,10 @@ __device__ __forceinline__ uint32_t stage_keys(const float* kb, uint32_t width, 
 // value finite (its product then a zero, which leaves the sum as it is): each
 // tile checks the masked keys and values it would leave out (finite, and no
 // dot product able to overflow) and otherwise attends query by query with
-// k_attention_rows' steps, as does a tile whose tokens differ in cache row or
-// length or are out of range.
+// k_attention_rows' steps, as does a tile with an entry out of range. Tokens of a
+// tile may differ in length (a position past a token's own length is no masked
+// one, and left out at any value); a tile of several cache rows is
+// k_attention_mixed's.
 
 // Query rows of a tile, at most; a workgroup's LDS at most (one workgroup of
 // eight waves a compute unit: two a SIMD, which the vector unit needs to issue
@@ -878,26 +910,26 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t m) {
 }
 
 // The attention of tokens [t0, t0 + count) (a tile of T), head h; false, with
-// nothing written, where the tokens do not share a cache row and length (or hold
-// an entry out of range), or a masked key or value could reach the host's
-// results. lds_floats: room for the scores.
+// nothing written, where the tile is mixed and not one of `others`' (whose
+// workgroups take it), or a masked key or value could reach the host's results.
+// lds_floats: room for the scores.
 template <int W>
 __device__ __forceinline__ bool attend_tile(const Attention& a, float* lds, uint32_t lds_floats, uint32_t T,
-                                            uint32_t t0, uint32_t count, uint32_t h, uint32_t tokens) {
+                                            uint32_t t0, uint32_t count, uint32_t h, uint32_t tokens, bool others) {
     __shared__ uint32_t found[TILE_WAVES][3];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // lane l: the entry of the tile's token l
     const uint32_t mine = t0 + min(lane, count - 1u);
     const int32_t row = a.table[3u * mine], last = a.table[3u * mine + 1u], length = a.table[3u * mine + 2u];
-    const int32_t row0 = __builtin_amdgcn_readfirstlane(row), held = __builtin_amdgcn_readfirstlane(length);
-    if (__builtin_amdgcn_ballot_w64(!entry_alike(a, mine, t0)) != 0) return false;
+    const int32_t row0 = __builtin_amdgcn_readfirstlane(row);
+    if (tile_mixed(a, t0, count)) return others;
     const uint32_t kv = h / (a.heads / a.kv_heads);
     const size_t base = ((size_t)row0 * a.kv_heads + kv) * a.capacity * W;
     const float* kb = a.keys + base;
     const float* vb = a.values + base;
 
-    // The masked positions: those some query does not see, up to the row's
-    // length.
+    // The masked positions: among those some query does not see, up to the
+    // longest length.
     int32_t least = last, most = last;
 #pragma unroll
     for (int s = 32; s >= 1; s >>= 1) {
@@ -906,6 +938,9 @@ __device__ __forceinline__ bool attend_tile(const Attention& a, float* lds, uint
     }
     least = __builtin_amdgcn_readfirstlane(least);
     most = __builtin_amdgcn_readfirstlane(most);
+    int32_t held = __builtin_amdgcn_readfirstlane(length);
+    for (uint32_t l = 1; __builtin_amdgcn_ballot_w64(length > held) != 0; ++l)
+        held = max(held, __builtin_amdgcn_readlane(length, l));
     if (least + 1 < held) {
         const uint32_t from = (uint32_t)(least + 1), masked = (uint32_t)held - from;
         uint32_t mk, mv, mq = 0;
@@ -1280,19 +1315,19 @@ __global__ __launch_bounds__(ROWS_THREADS, 2) void k_attention_rows(Attention a,
 }
 
 // The prompt kernel. Workgroup: a tile of T tokens (8, 16 or 32) and a head. A
-// tile that names more than one cache row or length, or whose masked positions
-// take part, goes query row by query row. lds_floats: the scores' room; kwaves:
-// attend_rows'.
+// mixed tile is left alone (`others`: k_attention_mixed takes it) or goes query
+// row by query row, as does one whose masked positions take part. lds_floats: the
+// scores' room; kwaves: attend_rows'.
 template <int W>
 __global__ __launch_bounds__(TILE_THREADS, 2) void k_attention_tile(Attention a, uint32_t tokens, uint32_t T, uint32_t tiles,
-                                                                    uint32_t lds_floats, uint32_t kwaves) {
+                                                                    uint32_t lds_floats, uint32_t kwaves, bool others) {
     static_assert(TILE_THREADS == ROWS_THREADS, "one workgroup runs both");
     extern __shared__ float4 lds4[];
     float* lds = reinterpret_cast<float*>(lds4);
     const uint32_t h = blockIdx.x % a.heads, order = blockIdx.x / a.heads;
     // a prompt's last tiles see most: they go first
     const uint32_t t0 = (tiles - 1u - order) * T, count = min(T, tokens - t0);
-    if (attend_tile<W>(a, lds, lds_floats, T, t0, count, h, tokens)) return;
+    if (attend_tile<W>(a, lds, lds_floats, T, t0, count, h, tokens, others)) return;
     for (uint32_t t = t0; t < t0 + count; ++t) {
         attend_rows<W, false, false>(a, RopeWrite{}, lds, kwaves, t, h);
         __syncthreads();
@@ -1341,15 +1376,27 @@ static hipError_t launch_rows(const Attention& a, const RopeWrite& r, uint32_t t
 // heads: 16 tokens 6.9 against 7.7, 32 tokens 11.7 against 8.3, 128 tokens 49
 // against 20, 512 tokens 469 against 65). The tiles' 16-byte loads need the
 // caches 16-byte aligned.
-constexpr uint32_t TILE_MIN_TOKENS = 16;
+//
+// Where the tokens may be of several cache rows, a tile of which is mixed, the
+// tiles are for at least four tokens a row (a step of as many sequences as
+// rows, or a few tokens of each: 24 sequences of up to 61 positions, 32 heads
+// take 8.5 us in k_attention, 44 in tiles whose workgroups, a compute unit each,
+// attend their tokens one after another; two tokens of each of 32 rows 31 us
+// against 46 with k_attention_mixed) and four workgroups of k_attention a
+// compute unit (k_attention_mixed's launch, k_attention's time first: 32 heads of
+// 64, no past, 24 tokens 7.6 and 11.3 us, 40 tokens 13.3 and 12.7; 9 heads, 72
+// tokens 10.0 and 12.5, 130 tokens 19.9 and 15.0; 16 heads of 128, 40 tokens 10.1
+// and 14.6, 72 tokens 22.2 and 18.7).
+constexpr uint32_t TILE_MIN_TOKENS = 16, TILE_ROW_TOKENS = 4;
 
-hipError_t launch_attention(const Attention& a, uint32_t tokens, int compute_units, hipStream_t stream) {
+hipError_t launch_attention(const Attention& a, uint32_t tokens, bool one_row, int compute_units, hipStream_t stream) {
     if (tokens == 0 || a.heads == 0) return hipSuccess;
     const size_t lds = attention_lds(a.width, a.capacity);
     const bool aligned = (((uintptr_t)a.keys | (uintptr_t)a.values) & 15u) == 0;
+    const bool others = !one_row && a.cache_rows > 1u;
     if (rows_fits(a, tokens, compute_units)) return launch_rows<false>(a, RopeWrite{}, tokens, stream);
-    if (tokens < TILE_MIN_TOKENS || 2u * (uint64_t)tokens * a.heads < 5u * (uint64_t)compute_units ||
-        (a.width != 64u && a.width != 128u) || !aligned) {
+    if (tokens < TILE_MIN_TOKENS || 2u * (uint64_t)tokens * a.heads < (others ? 8u : 5u) * (uint64_t)compute_units ||
+        (others && tokens < TILE_ROW_TOKENS * (uint64_t)a.cache_rows) || (a.width != 64u && a.width != 128u) || !aligned) {
         TMH_LAUNCH(k_attention, dim3(tokens * a.heads), dim3(256), lds, stream, a);
         return hipGetLastError();
     }
@@ -1370,9 +1417,15 @@ hipError_t launch_attention(const Attention& a, uint32_t tokens, int compute_uni
     const uint32_t floats = (uint32_t)(tile_lds / sizeof(float));
     const uint32_t kwaves = rows_kwaves(a, tile_lds);
     if (a.width == 64u)
-        TMH_LAUNCH(k_attention_tile<64>, dim3(work), dim3(TILE_THREADS), tile_lds, stream, a, tokens, T, tiles, floats, kwaves);
+        TMH_LAUNCH(k_attention_tile<64>, dim3(work), dim3(TILE_THREADS), tile_lds, stream, a, tokens, T, tiles, floats, kwaves,
+                   others);
     else
-        TMH_LAUNCH(k_attention_tile<128>, dim3(work), dim3(TILE_THREADS), tile_lds, stream, a, tokens, T, tiles, floats, kwaves);
+        TMH_LAUNCH(k_attention_tile<128>, dim3(work), dim3(TILE_THREADS), tile_lds, stream, a, tokens, T, tiles, floats, kwaves,
+                   others);
+    if (others) {
+        const uint32_t grid = (uint32_t)std::min<uint64_t>((uint64_t)tokens * a.heads, 3u * (uint64_t)compute_units);
+        TMH_LAUNCH(k_attention_mixed, dim3(grid), dim3(256), lds, stream, a, tokens, T);
+    }
     return hipGetLastError();
 }
 

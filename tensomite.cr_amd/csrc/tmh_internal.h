@@ -297,7 +297,8 @@ struct Attention {
 };
 size_t attention_lds(uint32_t width, uint32_t capacity);
 size_t attention_decode_lds(uint32_t width, uint32_t capacity);  // of launch_attention_decode
-hipError_t launch_attention(const Attention& a, uint32_t tokens, int compute_units, hipStream_t stream);
+// one_row: every token's table entry names the same cache row.
+hipError_t launch_attention(const Attention& a, uint32_t tokens, bool one_row, int compute_units, hipStream_t stream);
 // A decode step's attention with the RoPE and cache write of `r` fused: each
 // token is its cache row's one new position.
 hipError_t launch_attention_decode(const Attention& a, const RopeWrite& r, uint32_t tokens, int compute_units,

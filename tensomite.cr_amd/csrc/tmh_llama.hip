@@ -220,7 +220,7 @@ hipError_t forward_tokens(const Llama& m, const DeviceContext& ctx, uint32_t tok
                 e = tmh::launch_attention_decode(a, r, tokens, ctx.compute_units, ctx.stream);
             } else {
                 e = tmh::launch_rope_write(r, tokens, ctx.stream);
-                if (e == hipSuccess) e = tmh::launch_attention(a, tokens, ctx.compute_units, ctx.stream);
+                if (e == hipSuccess) e = tmh::launch_attention(a, tokens, true, ctx.compute_units, ctx.stream);
             }
         }
         if (e == hipSuccess && !quant_att) e = quantise(ctx, m.att, tokens, m.qn, a_att);
@@ -394,7 +394,7 @@ int tmh_attention(uint64_t q, uint32_t ldq, uint32_t tokens, uint32_t heads, uin
     if ((uint64_t)tokens * heads > 0x7fffffffull) return TMH_ERROR_SHAPE;
     tmh::Attention a{(const float*)q, ldq, (const float*)keys, (const float*)values, cache_rows, kv_heads, capacity,
                      width, heads, (const int32_t*)table, scale, (float*)dst, ld_dst, ctx.errors};
-    hipError_t e = tmh::launch_attention(a, tokens, ctx.compute_units, ctx.stream);
+    hipError_t e = tmh::launch_attention(a, tokens, false, ctx.compute_units, ctx.stream);
     if (e == hipSuccess) tmh::note_launch(ctx.index, 1, true);
     return code(e);
 }

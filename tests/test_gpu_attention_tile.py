@@ -73,6 +73,42 @@ def test_tiles_of_several_rows(dev):
     same(got, oracle.attention(q, k, v, table, scale))
 
 
+# Tokens of several cache rows in one call: as many sequences as tokens (a decode
+# step's), more query rows than a round of workgroups takes with every tile
+# mixed, and whole tiles beside mixed ones.
+@pytest.mark.parametrize("width", [64, 128])
+@pytest.mark.parametrize("tokens,heads,rows,run", [(24, 32, 24, 1), (200, 32, 5, 3), (150, 24, 4, 40)])
+def test_tokens_of_several_rows(dev, width, tokens, heads, rows, run):
+    print("several rows", width, tokens, heads, rows, run, flush=True)
+    capacity = 70
+    q, k, v = inputs(tokens, tokens, heads, 8, width, capacity, rows=rows)
+    rng = np.random.default_rng(tokens)
+    table = []
+    for t in range(tokens):
+        length = int(rng.integers(1, capacity + 1))
+        table.append((t // run % rows, int(rng.integers(0, length)), length))
+    got, scale = attend(dev, q, k, v, table)
+    dev.sync()
+    same(got, oracle.attention(q, k, v, table, scale))
+
+
+# Tokens of one row with a length each: a token does not see what lies past its
+# own length, masked or not, whatever the others see of it.
+@pytest.mark.parametrize("width", [64, 128])
+@pytest.mark.parametrize("beyond", [1.0, np.nan, np.inf])
+def test_tiles_of_own_lengths(dev, width, beyond):
+    print("own lengths", width, beyond, flush=True)
+    tokens, heads, capacity, past = 100, 16, 160, 40
+    q, k, v = inputs(17, tokens, heads, 8, width, capacity)
+    v[0, 3, past + 60, 5] = beyond
+    k[0, 2, past + 75, 9] = beyond
+    table = [(0, past + t, min(capacity, past + t + 1 + (t % 7) * 3)) for t in range(tokens)]
+    with np.errstate(all="ignore"):
+        got, scale = attend(dev, q, k, v, table)
+        dev.sync()
+        same(got, oracle.attention(q, k, v, table, scale))
+
+
 def test_tile_entry_out_of_range(dev):
     # the entry's token gets zeros and a report, the others their attention
     tokens, heads, capacity = 64, 16, 64
