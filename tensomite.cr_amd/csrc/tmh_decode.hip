@@ -1848,10 +1848,25 @@ __global__ __launch_bounds__(256) void k_attention_decode(Attention a, RopeWrite
     emit(l.out, out, width, a.act, t, h, a.heads);
 }
 
-hipError_t launch_attention_decode(const Attention& a, const RopeWrite& r, uint32_t tokens, int compute_units,
+// Head width 64: k_attention_decode's chunks hold 256 positions, all of which are on
+// their way from its start. One chunk: no slower at any number of rows (a step of
+// the 1.7B shape, k_attention_decode's time first: one row of 128 positions 823 and
+// 822 us, of 240 829 and 836, of 260 874 and 850; eight rows of 128 1369 and 1387, of
+// 240 1423 and 1475). Two: faster on a nearly full chip (eight rows of 32 heads of
+// 260 positions 1481 and 1498, of 500 1628 and 1648, of 640 1751 and 1751; six rows
+// of 320 2164 and 2168, of 500 2261 and 2247; four of 260 1354 and 1337). Width 128:
+// k_attention_rows from the first position (one row of 16 heads, 16 layers: at 8
+// positions 494 and 480, at 240 617 and 553).
+bool attention_decode_rows(const Attention& a, uint32_t tokens, uint32_t longest, int compute_units) {
+    if (!rows_fits(a, tokens, compute_units)) return false;
+    const bool full = 4u * (uint64_t)tokens * a.heads > 3u * (uint64_t)compute_units;
+    return a.width != 64u || longest > (full ? 512u : 256u);
+}
+
+hipError_t launch_attention_decode(const Attention& a, const RopeWrite& r, uint32_t tokens, bool by_rows,
                                    hipStream_t stream) {
     if (tokens == 0 || a.heads == 0) return hipSuccess;
-    if (rows_fits(a, tokens, compute_units)) return launch_rows<true>(a, r, tokens, stream);
+    if (by_rows) return launch_rows<true>(a, r, tokens, stream);
     const size_t lds = attention_decode_lds(a.width, a.capacity);
     TMH_LAUNCH(k_attention_decode, dim3(tokens * a.heads), dim3(256), lds, stream, a, r);
     return hipGetLastError();

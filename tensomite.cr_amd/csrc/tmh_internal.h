@@ -299,9 +299,13 @@ size_t attention_lds(uint32_t width, uint32_t capacity);
 size_t attention_decode_lds(uint32_t width, uint32_t capacity);  // of launch_attention_decode
 // one_row: every token's table entry names the same cache row.
 hipError_t launch_attention(const Attention& a, uint32_t tokens, bool one_row, int compute_units, hipStream_t stream);
+// Whether a decode step of `tokens` rows, of which the longest sees `longest`
+// positions, goes by k_attention_rows rather than k_attention_decode.
+bool attention_decode_rows(const Attention& a, uint32_t tokens, uint32_t longest, int compute_units);
 // A decode step's attention with the RoPE and cache write of `r` fused: each
-// token is its cache row's one new position.
-hipError_t launch_attention_decode(const Attention& a, const RopeWrite& r, uint32_t tokens, int compute_units,
+// token is its cache row's one new position. by_rows: attention_decode_rows' answer
+// (either kernel takes any length).
+hipError_t launch_attention_decode(const Attention& a, const RopeWrite& r, uint32_t tokens, bool by_rows,
                                    hipStream_t stream);
 
 // RMSNorm then quantisation into `act`, one launch; for n a multiple of 32

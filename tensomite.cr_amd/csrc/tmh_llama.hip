@@ -73,8 +73,8 @@ struct Llama {
     std::vector<char> has_logits;  // whether row r's logits row holds its last forward's
     bool generating = false;       // the device state continues a generation
 
-    hipGraphExec_t graph = nullptr;
-    // The step graph is captured on this stream of the model's own, so that
+    hipGraphExec_t graph[2] = {nullptr, nullptr};  // the step's, by its attention (step_attend)
+    // A step graph is captured on this stream of the model's own, so that
     // no other call (another thread's product on the device's stream) can
     // enqueue into the capture; the graph then runs on the device's stream.
     hipStream_t capture = nullptr;
@@ -171,14 +171,26 @@ hipError_t residual(const Llama& m, const DeviceContext& ctx, const uint8_t* w, 
     return e == hipSuccess ? tmh::launch_add(m.x[cur], m.o_out, m.x[cur], rows * W, ctx.stream) : e;
 }
 
+// How a forward attends: a prompt's tokens, or a step in which every token is its
+// cache row's one new position (a decode step, or a forward of one id), its
+// RoPE and cache write inside the attention launch, by k_attention_decode or
+// k_attention_rows.
+enum class Attend { PROMPT, STEP, STEP_ROWS };
+
+// A step's, of `tokens` rows of which the longest sees `longest` positions.
+Attend step_attend(const Llama& m, const DeviceContext& ctx, uint32_t tokens, uint32_t longest) {
+    tmh::Attention a{};
+    a.keys = m.keys, a.values = m.values;
+    a.capacity = m.capacity, a.width = (uint32_t)m.c.head_width, a.heads = (uint32_t)m.c.heads;
+    return tmh::attention_decode_rows(a, tokens, longest, ctx.compute_units) ? Attend::STEP_ROWS : Attend::STEP;
+}
+
 // The forward of `tokens` ids already on the device (m.ids), whose slots
 // and attention entries are on the device too; then the final norm and the
 // head over `final_rows` rows from row `final_from`, into logits rows from
-// `logits_row`. With `decode`, every token is its cache row's one new position
-// (a decode step, or a forward of one id), and its RoPE and cache write run
-// inside the attention launch.
+// `logits_row`.
 hipError_t forward_tokens(const Llama& m, const DeviceContext& ctx, uint32_t tokens, uint32_t final_from,
-                          uint32_t final_rows, uint32_t logits_row, bool decode) {
+                          uint32_t final_rows, uint32_t logits_row, Attend attend) {
     const tmh::TreeFold order(m.mode == TMH_MODE_UNORDERED);
     const tmh_llama_config& c = m.c;
     const uint32_t W = (uint32_t)c.width, H = (uint32_t)c.hidden, hw = (uint32_t)c.head_width;
@@ -216,8 +228,8 @@ hipError_t forward_tokens(const Llama& m, const DeviceContext& ctx, uint32_t tok
                          (uint32_t)c.heads, m.table, scale, m.att, m.qn, ctx.errors,
                          quant_att ? a_att : tmh::Activations{}};
         if (e == hipSuccess) {
-            if (decode) {
-                e = tmh::launch_attention_decode(a, r, tokens, ctx.compute_units, ctx.stream);
+            if (attend != Attend::PROMPT) {
+                e = tmh::launch_attention_decode(a, r, tokens, attend == Attend::STEP_ROWS, ctx.stream);
             } else {
                 e = tmh::launch_rope_write(r, tokens, ctx.stream);
                 if (e == hipSuccess) e = tmh::launch_attention(a, tokens, true, ctx.compute_units, ctx.stream);
@@ -287,14 +299,17 @@ hipError_t choose(const Llama& m, const DeviceContext& ctx) {
 
 // One decode step of every row from the device-held state: run each row's
 // chosen id, choose the next, log it and move the row on.
-hipError_t decode_step(const Llama& m, const DeviceContext& ctx) {
-    hipError_t e = forward_tokens(m, ctx, m.rows, 0, m.rows, 0, true);
+hipError_t decode_step(const Llama& m, const DeviceContext& ctx, Attend attend) {
+    hipError_t e = forward_tokens(m, ctx, m.rows, 0, m.rows, 0, attend);
     return e == hipSuccess ? choose(m, ctx) : e;
 }
 
 int run_step(Llama& m, const DeviceContext& ctx, bool graph) {
-    if (!graph) return code(decode_step(m, ctx));
-    if (!m.graph) {
+    const uint32_t held = (uint32_t)*std::max_element(m.length.begin(), m.length.end());
+    const Attend attend = step_attend(m, ctx, m.rows, held + 1u);
+    if (!graph) return code(decode_step(m, ctx, attend));
+    hipGraphExec_t& exec = m.graph[attend == Attend::STEP_ROWS];
+    if (!exec) {
         if (!m.capture) {
             hipError_t e = hipStreamCreateWithFlags(&m.capture, hipStreamNonBlocking);
             if (e != hipSuccess) {
@@ -307,21 +322,21 @@ int run_step(Llama& m, const DeviceContext& ctx, bool graph) {
         hipGraph_t g = nullptr;
         hipError_t e = hipStreamBeginCapture(cap.stream, hipStreamCaptureModeThreadLocal);
         if (e != hipSuccess) return code(e);
-        hipError_t step = decode_step(m, cap);
+        hipError_t step = decode_step(m, cap, attend);
         e = hipStreamEndCapture(cap.stream, &g);
         if (step != hipSuccess) {
             if (g) (void)hipGraphDestroy(g);
             return code(step);
         }
         if (e != hipSuccess) return code(e);
-        e = hipGraphInstantiate(&m.graph, g, nullptr, nullptr, 0);
+        e = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
         if (e != hipSuccess) {
-            m.graph = nullptr;
+            exec = nullptr;
             return code(e);
         }
     }
-    return code(hipGraphLaunch(m.graph, ctx.stream));
+    return code(hipGraphLaunch(exec, ctx.stream));
 }
 
 Llama* model_of(uint64_t handle, const DeviceContext& ctx, int* err) {
@@ -609,7 +624,8 @@ int tmh_llama_forward(uint64_t model, uint32_t row, const int32_t* ids, uint32_t
     // generation starts from.
     const uint32_t logits_row = last_only ? row : 0u;
     if (e == hipSuccess)
-        e = forward_tokens(*m, ctx, count, last_only ? count - 1u : 0u, final_rows, logits_row, count == 1u);
+        e = forward_tokens(*m, ctx, count, last_only ? count - 1u : 0u, final_rows, logits_row,
+                           count == 1u ? step_attend(*m, ctx, 1, (uint32_t)past + 1u) : Attend::PROMPT);
     if (e != hipSuccess) return code(e);
     tmh::note_launch(ctx.index, 0, true);
     m->length[row] = past + (int32_t)count;
@@ -727,11 +743,13 @@ int tmh_llama_set_mode(uint64_t model, uint32_t mode) {
     Llama* m = model_of(model, ctx, &err);
     if (!m) return err;
     if (mode != TMH_MODE_AUTO && mode != TMH_MODE_UNORDERED) return TMH_ERROR_INVALID_VALUE;
-    if (mode != m->mode && m->graph) {
-        // the captured step holds the old mode's kernel arguments
+    if (mode != m->mode && (m->graph[0] || m->graph[1])) {
+        // the captured steps hold the old mode's kernel arguments
         (void)hipStreamSynchronize(ctx.stream);
-        (void)hipGraphExecDestroy(m->graph);
-        m->graph = nullptr;
+        for (hipGraphExec_t& exec : m->graph) {
+            if (exec) (void)hipGraphExecDestroy(exec);
+            exec = nullptr;
+        }
     }
     m->mode = mode;
     return TMH_SUCCESS;
@@ -742,7 +760,8 @@ int tmh_llama_destroy(uint64_t model) {
     DeviceContext ctx;
     Llama* m = (Llama*)model;
     if (tmh::device_context(&ctx, false) == TMH_SUCCESS) (void)hipStreamSynchronize(ctx.stream);
-    if (m->graph) (void)hipGraphExecDestroy(m->graph);
+    for (hipGraphExec_t exec : m->graph)
+        if (exec) (void)hipGraphExecDestroy(exec);
     if (m->capture) (void)hipStreamDestroy(m->capture);
     if (m->memory) (void)hipFree(m->memory);
     if (m->owned) (void)hipFree(m->owned);

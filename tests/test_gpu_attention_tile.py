@@ -227,3 +227,27 @@ def test_prompt_tiles_quantised(dev, head_width, heads, tokens, capacity):
     want = oracle.Llama(config, weights).forward([int(i) for i in ids])
     got = th.HIPLlama(dev, config, weights, max_tokens=tokens).forward(ids)
     same(got, want)
+
+
+# Decode steps on both sides of the lengths at which the step's attention kernel
+# changes (256 positions of the longest row, 512 where the workgroups nearly fill
+# the chip), the shorter rows far from them: tokens from step graphs of either
+# kernel (the second time both captured), and eager ones.
+@pytest.mark.parametrize("rows,heads,longest", [(2, 4, 250), (8, 32, 250), (8, 32, 506)])
+def test_steps_across_the_attention_kernels(dev, rows, heads, longest):
+    from llama_fixtures import random_llama
+    print("steps", rows, heads, longest, flush=True)
+    config = dict(layers=2, width=64, heads=heads, kv_heads=4, head_width=64, hidden=64, vocab=96,
+                  context=600, eps=1e-5, theta=10000.0, kind="Q8_0")
+    weights = random_llama(config, seed=longest, std=0.2)
+    rng = np.random.default_rng(longest)
+    prompts = [[int(i) for i in rng.integers(0, 96, max(1, longest - 80 * r))] for r in range(rows)]
+    cpu = oracle.Llama(config, weights)
+    want = [cpu.generate(p, 12) for p in prompts]
+    model = th.HIPLlama(dev, config, weights, rows=rows, max_tokens=512)
+    for graph in (True, True, False):
+        for r, p in enumerate(prompts):
+            model.reset(r)
+            model.forward(p, row=r, last_only=True)
+        got = model.generate(12, graph=graph)
+        assert [list(t) for t in got] == want, graph
