@@ -3612,28 +3612,28 @@ static bool few_fits(const uint8_t* w, const Activations& act, uint32_t kind, ui
 }
 
 // A ring of 3 stage buffers leaves LDS for two workgroups a compute unit
-// (wide products: more than 256 workgroups; Q4_0 and Q4_1). Narrow ones have a
-// compute unit to themselves: stages of 32 blocks in a ring of 3 where the two
+// (wide products, of more workgroups than compute units; Q4_0 and Q4_1). Narrow
+// ones have a compute unit to themselves: stages of 32 blocks in a ring of 3 where the two
 // Q4 formats' rows are whole such stages (Q8_0's do not fit; a stage's time is
 // mostly its latencies and its barrier: 16 x 8192 -> 2048 Q4_1 16.1 us a call
 // with stages of 16, 13.9 with 32; 12 x 2048 -> 2048 Q4_0 8.1 with either), else
 // stages of 16 in a ring of 6. UNORDERED's sums go by stages of 16 always.
 template <int KIND>
 static hipError_t launch_few(const uint8_t* w, Activations act, float* dst, const float* bias, uint32_t bias_ld,
-                             uint32_t rows, uint32_t n, uint32_t k, hipStream_t stream) {
+                             uint32_t rows, uint32_t n, uint32_t k, int compute_units, hipStream_t stream) {
     const uint32_t grid = (n + FEW_COLS - 1u) / FEW_COLS;
-    const bool tree = tree_fold();
+    const bool tree = tree_fold(), wide = grid > (uint32_t)compute_units;
     if constexpr (KIND != 0) {
-        if (grid <= 256u && !tree && (k >> 5) % 32u == 0) {
+        if (!wide && !tree && (k >> 5) % 32u == 0) {
             TMH_LAUNCH((k_matmul_few<KIND, 3, 32, false>), dim3(grid), dim3(FEW_THREADS), 0, stream, w, act, dst,
                        bias, bias_ld, rows, n, k);
             return hipGetLastError();
         }
     }
-    if (grid > 256u && tree)
+    if (wide && tree)
         TMH_LAUNCH((k_matmul_few<KIND, 3, 16, true>), dim3(grid), dim3(FEW_THREADS), 0, stream, w, act, dst, bias,
                    bias_ld, rows, n, k);
-    else if (grid > 256u)
+    else if (wide)
         TMH_LAUNCH((k_matmul_few<KIND, 3, 16, false>), dim3(grid), dim3(FEW_THREADS), 0, stream, w, act, dst, bias,
                    bias_ld, rows, n, k);
     else if (tree)
@@ -3646,11 +3646,12 @@ static hipError_t launch_few(const uint8_t* w, Activations act, float* dst, cons
 }
 
 static hipError_t launch_few_kind(uint32_t kind, const uint8_t* w, Activations act, float* dst, const float* bias,
-                                  uint32_t bias_ld, uint32_t rows, uint32_t n, uint32_t k, hipStream_t stream) {
+                                  uint32_t bias_ld, uint32_t rows, uint32_t n, uint32_t k, int compute_units,
+                                  hipStream_t stream) {
     switch (kind) {
-    case 0: return launch_few<0>(w, act, dst, bias, bias_ld, rows, n, k, stream);
-    case 1: return launch_few<1>(w, act, dst, bias, bias_ld, rows, n, k, stream);
-    default: return launch_few<2>(w, act, dst, bias, bias_ld, rows, n, k, stream);
+    case 0: return launch_few<0>(w, act, dst, bias, bias_ld, rows, n, k, compute_units, stream);
+    case 1: return launch_few<1>(w, act, dst, bias, bias_ld, rows, n, k, compute_units, stream);
+    default: return launch_few<2>(w, act, dst, bias, bias_ld, rows, n, k, compute_units, stream);
     }
 }
 
@@ -3708,7 +3709,7 @@ hipError_t launch_block_matmul(uint32_t kind, uint32_t mode, const uint8_t* w, A
         if (e != hipErrorInvalidValue) return e;
     }
     if (autoish && few_fits(w, act, kind, rows, k))
-        return launch_few_kind(kind, w, act, dst, bias, 0, rows, n, k, stream);
+        return launch_few_kind(kind, w, act, dst, bias, 0, rows, n, k, compute_units, stream);
     if (matrix) return launch_matrix(kind, false, w, act, dst, bias, 0, rows, n, k, compute_units, stream);
     const bool thread = mode == 1u /* THREAD */ || !fits;
     switch (kind) {
@@ -3730,7 +3731,8 @@ hipError_t launch_product_residual(uint32_t kind, const uint8_t* w, Activations 
     if (!lanes_fit(w, k)) return hipErrorInvalidValue;
     if (rows >= MATRIX_ROWS)
         return launch_matrix(kind, false, w, act, dst, residual, n, rows, n, k, compute_units, stream);
-    if (few_fits(w, act, kind, rows, k)) return launch_few_kind(kind, w, act, dst, residual, n, rows, n, k, stream);
+    if (few_fits(w, act, kind, rows, k))
+        return launch_few_kind(kind, w, act, dst, residual, n, rows, n, k, compute_units, stream);
     switch (kind) {
     case 0: return launch_lanes<0>(w, act, dst, residual, rows, n, k, compute_units, stream, n);
     case 1: return launch_lanes<1>(w, act, dst, residual, rows, n, k, compute_units, stream, n);
