@@ -6,6 +6,8 @@
 
 namespace tmh {
 
+namespace {
+
 // x · wᵀ for many activation rows on the int8 matrix cores, for k a multiple
 // of 256 and 16-byte aligned weights and activation parts. A wave computes
 // tiles of 32 activation rows x 32 outputs over the whole of k: per block, one
@@ -425,6 +427,8 @@ __device__ __forceinline__ void mx_product(uint8_t* lds, const uint8_t* __restri
             if (row < m) dst[(size_t)row * n + col] = acc[i][e];
         }
 }
+
+}  // namespace
 
 // FS waves share a group's tiles: each issues all the MFMAs and folds its part
 // of every tile's results (the parts as separate code: a wave's results are
