@@ -247,7 +247,7 @@ __device__ __forceinline__ float wave_top(float top) {
 // Floats of one staged chunk of values (positions × width), at most; two
 // are staged in turn, in what the LDS (160 KB a workgroup on gfx950) leaves
 // after q, the current key and value, the outputs and the scores. Small
-// chunks leave room for several workgroups a compute unit (prefill runs
+// chunks leave room for several workgroups a compute unit (k_attention runs
 // one per query row and head).
 constexpr uint32_t ATT_CHUNK_FLOATS = 4096;
 constexpr size_t ATT_LDS_LIMIT = 160u * 1024u;
@@ -1026,7 +1026,10 @@ __device__ __forceinline__ bool attend_tile(const Attention& a, float* lds, uint
 //
 // One query row and head a workgroup of eight waves, for launches of at most
 // one workgroup a compute unit (a decode step's sequences): what a compute unit
-// can pull from HBM bounds it, so its loads stay in flight throughout.
+// can pull from HBM bounds it, so eight waves have loads out at once. A wave by
+// itself waits for all of its own at each first use: the number of loads before
+// one differs from path to path (whole, part and no groups of values), and the
+// compiler's counted waits assume the fewest.
 //
 //   scores   each wave takes blocks of 4096 / W positions (every `kwaves`-th),
 //            the keys by direct loads into LDS of its own, no barriers
@@ -1038,10 +1041,12 @@ __device__ __forceinline__ bool attend_tile(const Attention& a, float* lds, uint
 //            registers); the waves form their products together and then add
 //            them in turn to the running sums handed on through LDS
 //
-// Eight sequences of 500 to 2001 positions, 32 heads of 64: 80.2 -> 49 us a launch (176
-// MB of keys and values: 3.6 TB/s); one of 2001 positions 64.6 -> 31, one of 201 with
-// 9 heads 11.4 -> 8.0. k_attention read a chunk of 64 positions at a time, a
-// round trip each.
+// Eight sequences of 500 to 2001 positions, 32 heads of 64: 81.0 -> 51.7 us a launch
+// (176 MB of keys and values: 3.4 TB/s); one of 2001 positions 64.6 -> 31, one of 201
+// with 9 heads 11.4 -> 7.8. k_attention read a chunk of 64 positions at a time, a
+// round trip each; up to about 30 positions its four waves start sooner (9 positions
+// of 32 heads 5.9 us against 6.25), which the host, whose table is on the device,
+// does not know.
 constexpr uint32_t ROWS_THREADS = 512, ROWS_WAVES = ROWS_THREADS / 64;
 constexpr size_t ROWS_LDS = 159u * 1024u;
 constexpr uint32_t ROWS_KEY_FLOATS = 16u * 260u;  // a block's keys: 16 KB, 1040 bytes a kilobyte
@@ -1849,18 +1854,14 @@ __global__ __launch_bounds__(256) void k_attention_decode(Attention a, RopeWrite
 }
 
 // Head width 64: k_attention_decode's chunks hold 256 positions, all of which are on
-// their way from its start. One chunk: no slower at any number of rows (a step of
-// the 1.7B shape, k_attention_decode's time first: one row of 128 positions 823 and
-// 822 us, of 240 829 and 836, of 260 874 and 850; eight rows of 128 1369 and 1387, of
-// 240 1423 and 1475). Two: faster on a nearly full chip (eight rows of 32 heads of
-// 260 positions 1481 and 1498, of 500 1628 and 1648, of 640 1751 and 1751; six rows
-// of 320 2164 and 2168, of 500 2261 and 2247; four of 260 1354 and 1337). Width 128:
-// k_attention_rows from the first position (one row of 16 heads, 16 layers: at 8
-// positions 494 and 480, at 240 617 and 553).
+// their way from its start, so it is no slower while one chunk holds the longest
+// row (a step of the 1.7B shape, k_attention_decode's time first: one row of 128
+// positions 823 and 825 us, of 240 830 and 835, of 260 880 and 851; eight rows of 32
+// heads of 128 1372 and 1387, of 240 1439 and 1461, of 260 1497 and 1484, of 384 1566
+// and 1571). Width 128: k_attention_rows from the first position (one row of 16
+// heads, 16 layers: at 8 positions 494 and 480, at 240 617 and 553).
 bool attention_decode_rows(const Attention& a, uint32_t tokens, uint32_t longest, int compute_units) {
-    if (!rows_fits(a, tokens, compute_units)) return false;
-    const bool full = 4u * (uint64_t)tokens * a.heads > 3u * (uint64_t)compute_units;
-    return a.width != 64u || longest > (full ? 512u : 256u);
+    return rows_fits(a, tokens, compute_units) && (a.width != 64u || longest > 256u);
 }
 
 hipError_t launch_attention_decode(const Attention& a, const RopeWrite& r, uint32_t tokens, bool by_rows,

@@ -27,10 +27,13 @@ namespace {
 // rounded by itself. Measured on this machine, a SIMD issues such an
 // instruction every 2.4 cycles with two waves or more to choose from and every
 // 4.8 with one, and its matrix and vector instructions take turns: 185 cycles a
-// Q8_0 tile and block at best. So every wave folds, two to four of them a SIMD,
-// and unpacks its own weights from the raw blocks in LDS (8 to 24 instructions
-// a block); k_matmul_mx, whose compute units hold one folding wave a SIMD and
-// one that repacks weights for it, remains for the sizes between.
+// Q8_0 tile and block at best. So every wave folds, four of them a SIMD (128 x 128)
+// or two (64 x 128), and unpacks its own weights from the raw blocks in LDS (8 to 24
+// instructions a block). The 32 x 32 tiles are for products that would leave the
+// chip idle otherwise: their four waves, one a SIMD and so at half that rate,
+// share a tile's fold and each repeat its MFMAs and unpacking. k_matmul_mx, whose
+// compute units hold one folding wave a SIMD and one that repacks weights for it,
+// remains for the sizes between.
 //
 // The k axis goes in stages of 8 blocks through a ring of LDS buffers, one
 // workgroup barrier a stage, every byte brought by direct loads (16 bytes a

@@ -229,10 +229,10 @@ def test_prompt_tiles_quantised(dev, head_width, heads, tokens, capacity):
     same(got, want)
 
 
-# Decode steps on both sides of the lengths at which the step's attention kernel
-# changes (256 positions of the longest row, 512 where the workgroups nearly fill
-# the chip), the shorter rows far from them: tokens from step graphs of either
-# kernel (the second time both captured), and eager ones.
+# Decode steps on both sides of the length at which the step's attention kernel
+# changes (256 positions of the longest row), the shorter rows far from it: tokens
+# from step graphs of either kernel (the second time both captured), and eager
+# ones.
 @pytest.mark.parametrize("rows,heads,longest", [(2, 4, 250), (8, 32, 250), (8, 32, 506)])
 def test_steps_across_the_attention_kernels(dev, rows, heads, longest):
     from llama_fixtures import random_llama
