@@ -1,7 +1,9 @@
-"""Attention over many tokens (the prompt tiles) against the oracle, bit for
-bit: tile sizes 8, 16 and 32, partial tiles, a past, passes of fewer queries
-than a tile, head widths 64 and 128, tiles of several cache rows, and masked
-keys and values that reach the host's results."""
+"""Attention over many tokens (the prompt tiles) and over a step's few query rows
+against the oracle, bit for bit: tile sizes 8, 16 and 32, partial tiles, a past,
+passes of fewer queries than a tile, head widths 64 and 128, tokens of several
+cache rows or lengths, masked keys and values that reach the host's results, the
+tiles' outputs quantised in the decoder, and its steps on both sides of the
+length at which their kernel changes."""
 import sys
 
 import numpy as np
