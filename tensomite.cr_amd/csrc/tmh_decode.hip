@@ -1044,9 +1044,7 @@ __device__ __forceinline__ bool attend_tile(const Attention& a, float* lds, uint
 // Eight sequences of 500 to 2001 positions, 32 heads of 64: 81.0 -> 51.7 us a launch
 // (176 MB of keys and values: 3.4 TB/s); one of 2001 positions 64.6 -> 31, one of 201
 // with 9 heads 11.4 -> 7.8. k_attention read a chunk of 64 positions at a time, a
-// round trip each; up to about 30 positions its four waves start sooner (9 positions
-// of 32 heads 5.9 us against 6.25), which the host, whose table is on the device,
-// does not know.
+// round trip each.
 constexpr uint32_t ROWS_THREADS = 512, ROWS_WAVES = ROWS_THREADS / 64;
 constexpr size_t ROWS_LDS = 159u * 1024u;
 constexpr uint32_t ROWS_KEY_FLOATS = 16u * 260u;  // a block's keys: 16 KB, 1040 bytes a kilobyte
@@ -1312,11 +1310,88 @@ __device__ __forceinline__ void attend_rows(const Attention& a, const RopeWrite&
     emit(sums, out, W, a.act, t, h, a.heads);
 }
 
+// attend_rows of a row that fits one block of 64 positions (n of them, head width
+// 64), by one wave: nothing to hand on, no barriers. 32 heads, the eight waves' time
+// first: 9 positions 6.25 -> 4.6 us (k_attention 6.0), 21 positions 6.6 -> 4.5, 63
+// 7.4 -> 5.9; the look at the length costs longer rows 0.05 us.
+__device__ __forceinline__ void attend_block(const Attention& a, float* lds, uint32_t t, uint32_t h, int32_t row,
+                                             int32_t last, uint32_t n) {
+    constexpr uint32_t W = 64, P = 64;
+    const uint32_t lane = threadIdx.x;
+    const size_t base = ((size_t)row * a.kv_heads + h / (a.heads / a.kv_heads)) * a.capacity * W;
+    const float* vp = a.values + base + lane;
+    float* sums = lds;
+    float* sc = lds + W;
+    float* keys = sc + P;
+    float x[W / 16];
+#pragma unroll
+    for (int j = 0; j < (int)W / 16; ++j) x[j] = a.q[(size_t)t * a.ldq + (size_t)h * W + 16u * j + (lane & 15u)];
+    stage_keys<1>(a.keys + base, W, 0, n, lds_address(keys), 0);
+    float v[P];
+#pragma unroll
+    for (uint32_t g = 0; g < P; g += 16u) {
+        if (g >= n) break;
+#pragma unroll
+        for (uint32_t i = g; i < g + 16u; ++i) v[i] = i < n ? vp[(size_t)i * W] : 0.0f;
+    }
+    wait_vm_lds<0>();
+    asm volatile("" ::: "memory");
+    const uint32_t pl = 4u * (lane % 16u) + lane / 16u;  // tile_scores' lanes
+    const float4* k4 = reinterpret_cast<const float4*>(keys + att_key_at(pl * W));
+    float4 k[W / 4];
+#pragma unroll
+    for (uint32_t c = 0; c < W / 4u; ++c) k[c] = k4[c];
+    float dot = 0.0f;
+    add_key_columns<W>(dot, x, k);
+    float s = dot * a.scale;
+    if ((int32_t)pl > last) s = s + -__builtin_inff();  // attend_rows' mask
+    const float low = -__builtin_inff();
+    float top = wave_highest(pl < n && s > low ? s : low);
+    const float first = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(s)));
+    if (first != first) top = first;  // the host's top is a NaN at position 0
+    const float e = pl < n ? maths_exp(s - top) : 0.0f;
+    sc[pl] = e;
+    asm volatile("" ::: "memory");  // (a wave's LDS operations take effect in order)
+    const float total = ordered_sum_by_wave<false, 8>(sc, P);
+    sc[pl] = e / total;
+    asm volatile("" ::: "memory");
+    float acc = 0.0f;
+#pragma unroll
+    for (uint32_t g = 0; g < P; g += 16u) {
+        if (g >= n) break;
+        float prod[16];
+#pragma unroll
+        for (uint32_t i = 0; i < 16u; i += 4u) {
+            const float4 w4 = *reinterpret_cast<const float4*>(sc + g + i);
+            prod[i] = w4.x * v[g + i];
+            prod[i + 1u] = w4.y * v[g + i + 1u];
+            prod[i + 2u] = w4.z * v[g + i + 2u];
+            prod[i + 3u] = w4.w * v[g + i + 3u];
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < 16u; ++i) acc += prod[i];
+    }
+    sums[lane] = acc;
+    asm volatile("" ::: "memory");
+    emit(sums, a.dst + (size_t)t * a.ld_dst + (size_t)h * W, W, a.act, t, h, a.heads);
+}
+
 template <int W, bool EARLY, bool ROPE>
 __global__ __launch_bounds__(ROWS_THREADS, 2) void k_attention_rows(Attention a, RopeWrite r, uint32_t kwaves) {
     extern __shared__ float4 lds4[];
-    const uint32_t t = blockIdx.x / a.heads;
-    attend_rows<W, EARLY, ROPE>(a, r, reinterpret_cast<float*>(lds4), kwaves, t, blockIdx.x - t * a.heads);
+    float* lds = reinterpret_cast<float*>(lds4);
+    const uint32_t t = blockIdx.x / a.heads, h = blockIdx.x - t * a.heads;
+    if constexpr (W == 64 && !ROPE) {
+        // (an entry out of range is attend_rows')
+        const int32_t row = a.table[3u * t], last = a.table[3u * t + 1u], length = a.table[3u * t + 2u];
+        if (__builtin_expect(length > 0 && length <= 64 && length <= (int32_t)a.capacity && row >= 0 &&
+                                 row < (int32_t)a.cache_rows && last >= 0 && last < length,
+                             0)) {
+            if (threadIdx.x < 64u) attend_block(a, lds, t, h, row, last, (uint32_t)length);
+            return;
+        }
+    }
+    attend_rows<W, EARLY, ROPE>(a, r, lds, kwaves, t, h);
 }
 
 // The prompt kernel. Workgroup: a tile of T tokens (8, 16 or 32) and a head. A

@@ -175,6 +175,44 @@ def test_few_query_rows(dev, width, capacity, lengths):
         same(got, oracle.attention(q, k, v, table, scale))
 
 
+# Rows of one block of 64 positions (one wave's): groups of 16 whole and partial, the
+# causal end before the length, a NaN first score, values that are not finite seen and
+# masked, an entry out of range beside them; and in the decoder, quantised.
+def test_rows_of_one_block(dev):
+    lengths = [1, 2, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65]
+    q, k, v = inputs(3, len(lengths), 8, 2, 64, 70, rows=len(lengths))
+    k[4, 1, 0, 7] = np.nan
+    v[6, 0, 31, 3] = np.inf
+    k[8, 1, 46, 2] = -np.inf
+    v[9, 1, 40, 5] = np.nan
+    for seen in (1.0, 0.6):
+        table = [(i, max(0, int(n * seen) - 1), n) for i, n in enumerate(lengths)]
+        with np.errstate(all="ignore"):
+            got, scale = attend(dev, q, k, v, table)
+            dev.sync()
+            want = oracle.attention(q, k, v, table, scale)
+        same(got, want)
+    table[3] = (3, 16, 16)
+    with np.errstate(all="ignore"):
+        got, _ = attend(dev, q, k, v, table)
+    with pytest.raises(th.ExecutionError):
+        dev.sync()
+    assert np.all(got[3] == 0)
+    keep = np.arange(len(lengths)) != 3
+    same(got[keep], want[keep])
+
+
+@pytest.mark.parametrize("tokens", [3, 16, 33, 64])
+def test_prompt_of_one_block_quantised(dev, tokens):
+    from llama_fixtures import random_llama
+    config = dict(layers=2, width=64, heads=4, kv_heads=2, head_width=64, hidden=64, vocab=96, context=80, eps=1e-5,
+                  theta=10000.0, kind="Q4_0")
+    weights = random_llama(config, seed=tokens, std=0.2)
+    ids = np.random.default_rng(tokens).integers(0, 96, tokens).astype(np.int32)
+    want = oracle.Llama(config, weights).forward([int(i) for i in ids])
+    same(th.HIPLlama(dev, config, weights, max_tokens=tokens).forward(ids), want)
+
+
 # Capacities whose scores fill the workgroup's LDS: the last one with room for
 # two waves' keys, the first without, the first without room for one's, and the
 # largest the entry point takes.
